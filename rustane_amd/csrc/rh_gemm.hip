@@ -11,11 +11,11 @@
 // lane's accumulator then holds 4 consecutive output features of one token,
 // which makes the RoPE pairs (2i, 2i+1) and 16-byte fp32 stores lane-local.
 //
-// Tile policy: DTile (below) -- both operands in fragment order in HBM, moved
+// Tile policies: DTile (below) -- both operands in fragment order in HBM, moved
 // global -> LDS by DMA through a 4-stage (192x256: 5-stage) pipeline of 32-wide k slices,
-// 32x32x16 MFMA (16x16x32 for the 8-wave tiles but 256x256) on fragments
-// double-buffered in registers (256x256 keeps 32x32x16: its 16x16x32 form
-// spills).  Instantiated as
+// 32x32x16 MFMA (16x16x32 for the 8-wave tiles) on fragments double-buffered
+// in registers -- and PTile, the same operands with the block's two halves
+// taking turns at the matrix pipes (8-wave 256x256 and 256x128).  Instantiated as
 // 256x256 (8 waves of 128x64, or 4 waves of 128x128 with AGPR accumulators),
 // 256x128, 192x256, 192x128 and 128x128; a cost model picks one per shape.
 // Out-of-range rows are clamped, not predicated (they only feed accumulator
@@ -283,6 +283,136 @@ struct DTile {
                 step(t0 + 9, f1, f0, buf(4), buf(0));
             }
         }
+        // the trailing (unused) stage loads must land before the LDS is reused
+        __builtin_amdgcn_s_waitcnt(vm_wait(0));
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Ping-pong tile (PTile): the same operands, fragments and DMA as DTile, but
+// the block's 8 waves form two groups of 4 (one wave of each per SIMD) that
+// take turns.  While one group runs a stage's MFMAs with nothing else in its
+// instruction stream, the other reads its next fragments from LDS and issues
+// its share of the next DMA; a barrier swaps them.  DTile instead has both
+// waves of a SIMD do everything at once, and whenever the vector-memory queue
+// is full their in-order issue holds the MFMAs back: at 8192 x 4096 x 11008
+// its 256x256 tile keeps the matrix pipes 68% busy (1.60 GHz), this one 79%
+// (1.62 GHz), and what is left is the two barriers per stage and the
+// prologue and epilogue of each tile.  The part is power-limited at these
+// sizes, so the order of the MFMAs counts too: consecutive ones share one
+// operand (every other row of B tiles runs backwards: +1.5%), and handing the
+// matrix pipe over 4 MFMAs before the end of a stage (so that the two waves'
+// MFMAs mix) costs 6%.  Measured at M = 8192 (7B, us, DTile 256x256 -> this):
+// QKV 739 -> 623, W1|W3 1220 -> 1050, W2 623 -> 524, Wo 260 -> 225, logits
+// 1856 -> 1635; 4096 x 4096 x 22016 594 -> 487 (1.52 PFLOP/s).
+//
+// A stage is KD slices of 32 k.  NS stages ring in LDS: at stage t each wave
+// reads stage t, issues stage t + NS - 1 into the buffer stage t - 1 came
+// from, and waits for its own part of stage t + 1.  Group 1 runs one barrier
+// interval behind group 0, so group 0 fetches stage t in interval 2t and group
+// 1 in 2t + 1; stage t - 1 was last read in interval 2t - 1, before either
+// group refills its buffer, and both groups' parts of stage t + 1 have landed
+// by the barrier that ends interval 2t + 1.  Every wave executes the same
+// number of barriers (group 1 one extra at the start, group 0 at the end).
+// The small tiles gain nothing from this (their stages hold too few MFMAs
+// between barriers): 192x128 and 128x128 stay DTiles.  256x128 runs two k
+// slices a stage (32 MFMAs between barriers, as 256x256): 163 -> 157 us at
+// 2048 x 4096 x 11008, 132 -> 129 at 512 x 32000 x 4096.
+template <int WGN, int WGM, int NA_, int NB_, int KD, int NS_>
+struct PTile {
+    static_assert(WGN * WGM == 8 && NA_ % 2 == 0 && (NS_ == 3 || NS_ == 4), "8 waves, 3 or 4 stages");
+    static constexpr bool kM16 = true;
+    static constexpr int NA = NA_, NB = NB_, BN = 16 * NA * WGN, BM = 16 * NB * WGM, NT = 512;
+    static constexpr int FTN = NA / 2, FTM = NB / 2, KI = 32 * KD, NS = NS_;
+    static constexpr int NWF = BN / 16, NF = NWF + BM / 16, LPS = NF * KD / 8, SH = NF * KD * 512;
+    static_assert(NF * KD % 8 == 0, "the DMA of a stage splits evenly over the waves");
+    using Acc = Frag16<NA, NB>;
+    struct Smem {};
+    __device__ static int nw(int n0) { return n0 + ((threadIdx.x >> 6) % WGN) * 16 * NA; }
+    __device__ static int mw(int m0) { return m0 + ((threadIdx.x >> 6) / WGN) * 16 * NB; }
+    // s_waitcnt with vmcnt <= n; the same with lgkmcnt == 0
+    static constexpr int vm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+    static constexpr int vm_lgkm_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
+
+    __device__ static void run(const GemmArgs& a, int n0, int m0, int kb, int ke, Acc& acc, Smem&) {
+        __shared__ __attribute__((aligned(1024))) f16 st0[SH], st1[SH], st2[SH];
+        f16* st3 = st0;  // names no fourth buffer when NS == 3
+        if constexpr (NS > 3) {
+            __shared__ __attribute__((aligned(1024))) f16 st3s[SH];
+            st3 = st3s;
+        }
+        auto buf = [&](int s) -> f16* { return s == 0 ? st0 : s == 1 ? st1 : s == 2 ? st2 : st3; };
+        const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+        const int wn = wv % WGN, wm = wv / WGN, grp = wv >> 2;
+        // this wave's DMA units: u = wv * LPS + q over [weight fragments | activation fragments] x KD slices
+        const f16* gp[LPS];
+#pragma unroll
+        for (int q = 0; q < LPS; ++q) {
+            const int u = wv * LPS + q, f = u / KD, d = u % KD;
+            const int rb = f < NWF ? min((n0 >> 4) + f, ((a.N + 15) >> 4) - 1)
+                                   : min((m0 >> 4) + f - NWF, ((a.M + 15) >> 4) - 1);
+            gp[q] = (f < NWF ? a.W : a.X) + (size_t)rb * a.K * 16 + d * 512 + lane * 8;
+        }
+        auto dma = [&](int kt, f16* st, int q) {
+            __builtin_amdgcn_global_load_lds(
+                (const void*)(gp[q] + (size_t)kt * (512 * KD)),
+                (__attribute__((address_space(3))) void*)(st + (wv * LPS + q) * 512), 16, 0, 0);
+        };
+        const int ao = wn * NA * KD * 512 + 8 * lane, bo = (NWF + wm * NB) * KD * 512 + 8 * lane;
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) acc.v[i][j] = f32x4{};
+        // no wave may still read the stages from a previous call
+        __builtin_amdgcn_s_waitcnt(vm_lgkm_wait(63));
+        __builtin_amdgcn_s_barrier();
+        const int n = ke - kb;
+#pragma unroll
+        for (int p = 0; p < NS - 1; ++p)
+#pragma unroll
+            for (int q = 0; q < LPS; ++q) dma(kb + min(p, n - 1), buf(p), q);
+        __builtin_amdgcn_s_waitcnt(vm_wait((NS - 2) * LPS));
+        __builtin_amdgcn_s_barrier();
+        if (grp == 1) __builtin_amdgcn_s_barrier();
+        // Stage t from st; stage t + NS - 1 (clamped: past the end a reload of
+        // the last one that nobody reads) into refill.
+        auto stage = [&](int t, const f16* st, f16* refill) {
+            f16x8 fa[KD][NA], fb[KD][NB];
+            const int kt = kb + min(t + NS - 1, n - 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int d = 0; d < KD; ++d) {
+#pragma unroll
+                for (int j = 0; j < NB; ++j) fb[d][j] = *(const f16x8*)&st[bo + (j * KD + d) * 512];
+#pragma unroll
+                for (int i = 0; i < NA; ++i) fa[d][i] = *(const f16x8*)&st[ao + (i * KD + d) * 512];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = 0; q < LPS; ++q) dma(kt, refill, q);
+            __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_waitcnt(vm_lgkm_wait((NS - 2) * LPS));
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int d = 0; d < KD; ++d)
+#pragma unroll
+                for (int m = 0; m < NA * NB; ++m) {
+                    const int i = m / NB, j = i & 1 ? NB - 1 - m % NB : m % NB;
+                    acc.v[i][j] = mfma16(fa[d][i], fb[d][j], acc.v[i][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        for (int t0 = 0; t0 < n; t0 += NS) {
+            stage(t0, st0, buf(NS - 1));
+            if (t0 + 1 < n) stage(t0 + 1, st1, st0);
+            if (t0 + 2 < n) stage(t0 + 2, st2, st1);
+            if constexpr (NS > 3)
+                if (t0 + 3 < n) stage(t0 + 3, st3, st2);
+        }
+        if (grp == 0) __builtin_amdgcn_s_barrier();
         // the trailing (unused) stage loads must land before the LDS is reused
         __builtin_amdgcn_s_waitcnt(vm_wait(0));
     }
@@ -768,6 +898,9 @@ __global__ __launch_bounds__(Tl::NT + 64 * WG_SW) void gemm_wgrad_kernel(GemmArg
     }
 }
 
+using Tile256x256 = PTile<2, 4, 8, 4, 1, 4>;
+using Tile256x128 = PTile<4, 2, 4, 4, 2, 3>;
+
 template <int EPI>
 hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
     int cfg = a.force_cfg;
@@ -776,13 +909,16 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
         // tile FLOPs / that tile's per-CU rate.  The rates are fitted to MI355X
         // timings of every tile on 27 GEMM shapes of the 7B forward and
         // training step (M 512 - 8192, random fp16 operands; the picks land
-        // within 0.5% of the per-shape best in total); the estimate trades wave
+        // within 0.5% of the per-shape best in total; 256x256 and 256x128 refitted
+        // for the ping-pong tiles: at M = 8192 a 256x256 tile takes 1.20 times a
+        // 192x256 one's time for 1.33 times its work, at M = 512 1.09 times for a
+        // tile of W1|W3); the estimate trades wave
         // quantization (e.g. 172 vs 230 tiles at M = 512) against per-tile
         // efficiency.  Narrow outputs (Wo) and long K (W2) use stream-K
         // instead, when every block gets at least two 32-wide k-iterations.
         struct Cand { int cfg, bn, bm; float rate; };
-        constexpr Cand dp[] = {{GCFG_D8_256x256, 256, 256, 4.4f}, {GCFG_D8_192x256, 192, 256, 4.35f},
-                               {GCFG_D8_256x128, 256, 128, 3.6f}, {GCFG_D8_192x128, 192, 128, 3.7f},
+        constexpr Cand dp[] = {{GCFG_D8_256x256, 256, 256, 5.0f}, {GCFG_D8_192x256, 192, 256, 4.35f},
+                               {GCFG_D8_256x128, 256, 128, 3.75f}, {GCFG_D8_192x128, 192, 128, 3.7f},
                                {GCFG_D8_128x128, 128, 128, 3.0f}};
         const long long KT = a.K / 32;
         const int t256x128 = ((a.N + 255) / 256) * ((a.M + 127) / 128);
@@ -805,22 +941,21 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
             }
         }
     }
-    // The 8-wave 192x256, 192x128, 256x128 and 128x128 tiles run the
-    // 16x16x32 form: at M = 512 (7B) W1|W3 takes 84.5 us as 8-wave 16x16x32
-    // 192x256, against 87.8 as a 4-wave 16x16x32 tile and 91.4 as 8-wave
-    // 32x32x16; QKV 60.4 us as 8-wave 16x16x32 192x128 against 64.7 as 4-wave
-    // 32x32x16; the 8-wave 256x128 and 128x128 tiles are 0-12% and 1-6%
-    // faster in that form than their 32x32x16 twins on every shape timed.  The
-    // 4-wave 192x128 tile stays 32x32x16: the weight-gradient GEMMs need its
-    // two blocks per CU, which the 16x16x32 form's extra registers would
-    // cost; the 8-wave 256x256 tile spills in that form.
+    // The 8-wave 192x256, 192x128 and 128x128 tiles run the 16x16x32 form: at
+    // M = 512 (7B) W1|W3 takes 84.5 us as 8-wave 16x16x32 192x256, against 87.8
+    // as a 4-wave 16x16x32 tile and 91.4 as 8-wave 32x32x16; QKV 60.4 us as
+    // 8-wave 16x16x32 192x128 against 64.7 as 4-wave 32x32x16; the 8-wave
+    // 128x128 tile is 1-6% faster in that form than its 32x32x16 twin on every
+    // shape timed.  8-wave 256x256 and 256x128 are ping-pong tiles.  The
+    // 4-wave 192x128 tile stays 32x32x16 (in the 16x16x32 form its second
+    // block per CU would not fit the registers).
     switch (cfg) {
-        case GCFG_D8_256x256: return launch_tile<DTile<2, 4, 4, 2>, EPI>(a, false, st);
-        case GCFG_D8_256x256_SK: return launch_tile<DTile<2, 4, 4, 2>, EPI>(a, true, st);
+        case GCFG_D8_256x256: return launch_tile<Tile256x256, EPI>(a, false, st);
+        case GCFG_D8_256x256_SK: return launch_tile<Tile256x256, EPI>(a, true, st);
         case GCFG_D4_128x128: return launch_tile<DTile<2, 2, 2, 2>, EPI>(a, false, st);
         case GCFG_D4_128x128_SK: return launch_tile<DTile<2, 2, 2, 2>, EPI>(a, true, st);
-        case GCFG_D8_256x128: return launch_tile<DTile<4, 2, 2, 2, true>, EPI>(a, false, st);
-        case GCFG_D8_256x128_SK: return launch_tile<DTile<4, 2, 2, 2, true>, EPI>(a, true, st);
+        case GCFG_D8_256x128: return launch_tile<Tile256x128, EPI>(a, false, st);
+        case GCFG_D8_256x128_SK: return launch_tile<Tile256x128, EPI>(a, true, st);
         case GCFG_D4_256x256: return launch_tile<DTile<2, 2, 4, 4>, EPI>(a, false, st);
         case GCFG_D4_256x256_SK: return launch_tile<DTile<2, 2, 4, 4>, EPI>(a, true, st);
         case GCFG_D4_256x128: return launch_tile<DTile<2, 2, 4, 2>, EPI>(a, false, st);
@@ -871,7 +1006,9 @@ int split_count(const GemmArgs& a) {
 }
 
 // K >= 8192 (W2): 256x128 tiles as 8 waves of 16x16x32 (50.3 vs 52.9 us as 4
-// waves of 32x32x16 at 7B, M = 512); otherwise 128x128 (the two forms measure
+// waves of 32x32x16 at 7B, M = 512; the ping-pong 256x128 tile measures the
+// same there and loses at short prompts, whole 7B prefill of 45 tokens 4.23 ->
+// 4.34 ms); otherwise 128x128 (the two forms measure
 // the same there)
 hipError_t launch_split_any(const GemmArgs& a, int S, hipStream_t st) {
     return a.K >= 8192 ? launch_split<DTile<4, 2, 2, 2, true>>(a, S, st) : launch_split<DTile<2, 2, 2, 2>>(a, S, st);

@@ -42,15 +42,15 @@ struct GemmArgs {
     // launches otherwise.
     hipEvent_t prof_start, prof_stop;
 };
-// Tile configurations of the prefill GEMM (all: direct-to-LDS 4-stage
-// pipeline; waves x per-wave tile).
+// Tile configurations of the prefill GEMM (all: direct-to-LDS pipeline;
+// waves x per-wave tile).
 enum GemmCfg {
     GCFG_AUTO = 0,
-    GCFG_D8_256x256 = 6,     // 8 waves (128x64 each)
+    GCFG_D8_256x256 = 6,     // 8 waves (128x64 each), ping-pong, 16x16x32 MFMA
     GCFG_D8_256x256_SK = 7,  // ... stream-K
     GCFG_D4_128x128 = 8,     // 4 waves (64x64 each)
     GCFG_D4_128x128_SK = 9,
-    GCFG_D8_256x128 = 10,    // 8 waves (64x64 each), 16x16x32 MFMA
+    GCFG_D8_256x128 = 10,    // 8 waves (64x64 each), ping-pong, 16x16x32 MFMA
     GCFG_D8_256x128_SK = 11,
     GCFG_D4_256x256 = 12,    // 4 waves (128x128 each, accumulators in AGPRs)
     GCFG_D4_256x256_SK = 13,
