@@ -21,9 +21,9 @@ BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "librustane_hip.so")
 HARNESS = os.path.join(HERE, "librustane_gemm_harness.so")
 HARNESS_SOURCES = ["rh_gemm_harness.cpp"]
-HARNESS_DEPS = ["rh_gemm.hip", "rh_rowops.hip"]  # objects of SOURCES it links
+HARNESS_DEPS = ["rh_gemm.hip", "rh_skinny.hip", "rh_rowops.hip"]  # objects of SOURCES it links
 
-SOURCES = ["rh_gemm.hip", "rh_attn.hip", "rh_attn_bwd.hip", "rh_gemv.hip", "rh_rowops.hip", "rh_trainops.hip", "rh_optim.hip",
+SOURCES = ["rh_gemm.hip", "rh_skinny.hip", "rh_attn.hip", "rh_attn_bwd.hip", "rh_gemv.hip", "rh_rowops.hip", "rh_trainops.hip", "rh_optim.hip",
            "rh_runtime.cpp", "rh_train.cpp", "rh_data.cpp", "rh_sched.cpp", "rh_noalloc.cpp"]
 ARCH = "gfx950"
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -38,7 +38,9 @@ CFLAGS = [
 # every key block; with accumulators in AGPRs each rescale costs two copies
 # per register, so its MFMAs take the VGPR form (the GEMMs keep AGPRs: their
 # accumulators exceed the 256 architectural VGPRs).
-FILE_FLAGS = {"rh_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
+# The few-token GEMM's sums, rotated through AGPRs otherwise, stay in VGPRs too.
+FILE_FLAGS = {"rh_skinny.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
+              "rh_attn.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
               "rh_attn_bwd.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"]}
 
 

@@ -67,6 +67,16 @@ enum GemmCfg {
     GCFG_D8_128x128 = 26,    // 8 waves (64x32 each), 16x16x32 MFMA
     GCFG_D8_128x128_SK = 27,
 };
+// Few tokens (rh_skinny.hip): every weight row streamed once for all M <=
+// SKINNY_M tokens.  launch_gemm_skinny: EPI_F32, EPI_SWIGLU, EPI_QKV;
+// launch_gemm_skinny_split: S fp32 partials [M][N] at sk_part (1 <= S <=
+// skinny_splits(a)).  The line lies where the tile kernels take over: whole
+// 7B prefill takes 4.52 -> 3.62 ms at 64 tokens (past them a fifth token tile
+// would not leave room for the weights in flight; tile kernels 4.58 ms at 65).
+constexpr int SKINNY_M = 64;
+int skinny_splits(const GemmArgs& a);
+hipError_t launch_gemm_skinny(int epi, const GemmArgs& a, hipStream_t st);
+hipError_t launch_gemm_skinny_split(const GemmArgs& a, int S, hipStream_t st);
 // Floats of stream-K workspace any prefill GEMM needs.
 size_t gemm_sk_part_floats();
 hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t st);

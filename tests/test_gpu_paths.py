@@ -9,6 +9,8 @@ from rustane_amd.engine import ModelWeights
 
 from helpers import random_gammas, small_cfg
 from test_gpu_backward import _run
+from test_gpu_gemm_tiles import (CFGS, EPI_F32, EPI_QKV, EPI_SWIGLU, close, frag_pack, frag_unpack, lib,  # noqa: F401
+                                 operands, ptr, run, swiglu_ref, up16)
 
 pytestmark = pytest.mark.gpu
 
@@ -24,3 +26,73 @@ def test_embedding_gradient_of_repeated_tokens(orc):
     tok = rng.permutation(ids).reshape(2, 64).astype(np.uint32)
     tgt = rng.integers(0, cfg.vocab, size=tok.shape).astype(np.uint32)
     _run(orc, cfg, w, np.ascontiguousarray(tok), tgt)
+
+
+@pytest.mark.parametrize("K", [128, 256, 384, 640, 1152])
+@pytest.mark.parametrize("name", ["D8_256x256", "D8_256x256_SK", "D8_256x128", "D8_256x128_SK"])
+def test_ping_pong_step_counts(lib, name, K):  # noqa: F811
+    """k loops shorter than the stage ring, ending on each of its buffers."""
+    x, w, y = operands(21, 270, 520, K)
+    out = np.zeros((270, 520), np.float32)
+    run(lib, EPI_F32, CFGS[name], x, w, io=out)
+    close(out, y, 1e-5, f"{name} K {K}")
+
+
+# Few tokens: token tiles of 16 full and ragged, 64 and the first count past
+# it; every choice of row tiles per block (by N), ragged in N; fewer k chunks
+# than waves, more, and a remainder.  fp32 sums of K <= 1408 products: 1e-5 of
+# max|Y|; fp16 outputs one rounding: 2e-3.
+@pytest.mark.parametrize("M", [1, 16, 17, 45, 64, 65])
+@pytest.mark.parametrize("N,K", [(996, 128), (1000, 1152), (8204, 384)])
+def test_few_tokens_fp32(lib, M, N, K):  # noqa: F811
+    x, w, y = operands(22, M, N, K)
+    out = np.full((M, N), np.nan, np.float32)
+    run(lib, EPI_F32, 0, x, w, alpha=0.5, softcap=30.0, io=out)
+    close(out, 30.0 * np.tanh(0.5 * y / 30.0), 1e-5, f"M {M}")
+
+
+@pytest.mark.parametrize("M", [1, 33, 64])
+@pytest.mark.parametrize("F,K", [(128, 128), (4224, 256), (8320, 1408)])
+def test_few_tokens_swiglu(lib, M, F, K):  # noqa: F811
+    x, w, y = operands(23, M, 2 * F, K)
+    out16 = np.zeros(up16(M) * F, np.float16)
+    run(lib, EPI_SWIGLU, 0, x, w, out16=out16)
+    close(frag_unpack(out16, M, F), swiglu_ref(y)[0], 2e-3, f"M {M} F {F}")
+
+
+@pytest.mark.parametrize("B,S,H,hd", [(1, 5, 3, 64), (3, 16, 22, 128), (2, 31, 33, 128)])
+def test_few_tokens_qkv(lib, B, S, H, hd):  # noqa: F811
+    ctx, pos0, K, D = S + 9, 4, 256, H * hd
+    x, w, y = operands(24, B * S, 3 * D, K)
+    ang = np.random.default_rng(25).uniform(-np.pi, np.pi, (ctx, hd // 2))
+    rope = np.stack([np.cos(ang), np.sin(ang)], -1).astype(np.float32)
+    q, k, v = (np.zeros((B, H, n, hd), np.float16) for n in (S, ctx, ctx))
+    run(lib, EPI_QKV, 0, x, w, qkv=(B, S, H, hd, ctx, pos0, rope, q, k, v))
+    y = y.reshape(B, S, 3, H, hd).transpose(2, 0, 3, 1, 4)
+    c, s = (rope[pos0:pos0 + S, :, i].astype(np.float64) for i in (0, 1))
+
+    def rot(t):
+        e, o = t[..., 0::2], t[..., 1::2]
+        return np.stack([e * c - o * s, o * c + e * s], -1).reshape(t.shape)
+
+    close(q, rot(y[0]), 2e-3, "q")
+    close(k[:, :, pos0:pos0 + S], rot(y[1]), 2e-3, "k cache")
+    close(v[:, :, pos0:pos0 + S], y[2], 2e-3, "v cache")
+    assert not k[:, :, :pos0].any() and not k[:, :, pos0 + S:].any()
+
+
+@pytest.mark.parametrize("M", [1, 45, 64])
+@pytest.mark.parametrize("N,K", [(1024, 128), (1024, 1152), (2688, 1408), (8192, 640)])
+def test_few_tokens_residual_then_rmsnorm(lib, M, N, K):  # noqa: F811
+    eps, alpha = 1e-5, 0.25
+    x, w, y = operands(26, M, N, K)
+    rng = np.random.default_rng(27)
+    x0 = rng.standard_normal((M, N)).astype(np.float32)
+    gamma = rng.uniform(0.5, 1.5, N).astype(np.float32)
+    io, xn = x0.copy(), np.zeros(up16(M) * N, np.float16)
+    rc = lib.rhh_gemm_resid_norm(0, ptr(frag_pack(w)), ptr(frag_pack(x)), M, N, K, alpha, None, ptr(io), ptr(gamma),
+                                 eps, ptr(xn))
+    assert rc == 0
+    x1 = x0.astype(np.float64) + alpha * y
+    close(io, x1, 1e-5, "residual")
+    close(frag_unpack(xn, M, N), x1 / np.sqrt((x1 * x1).mean(1, keepdims=True) + eps) * gamma, 2e-3, "rmsnorm")
