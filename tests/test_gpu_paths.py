@@ -5,9 +5,10 @@ same path."""
 import numpy as np
 import pytest
 
+from rustane_amd import hip_bridge as hb
 from rustane_amd.engine import ModelWeights
 
-from helpers import random_gammas, small_cfg
+from helpers import LOGIT_ATOL, random_gammas, small_cfg, tokens_uniform
 from test_gpu_backward import _run
 from test_gpu_gemm_tiles import (CFGS, EPI_F32, EPI_QKV, EPI_SWIGLU, close, frag_pack, frag_unpack, lib,  # noqa: F401
                                  operands, ptr, run, swiglu_ref, up16)
@@ -96,3 +97,25 @@ def test_few_tokens_residual_then_rmsnorm(lib, M, N, K):  # noqa: F811
     x1 = x0.astype(np.float64) + alpha * y
     close(io, x1, 1e-5, "residual")
     close(frag_unpack(xn, M, N), x1 / np.sqrt((x1 * x1).mean(1, keepdims=True) + eps) * gamma, 2e-3, "rmsnorm")
+
+
+def _decode_matches_forward(cfg, B, p0, steps, seed, max_ctx=0):
+    """Teacher-forced decode logits equal the forward's at every position."""
+    w = random_gammas(ModelWeights.normal(cfg, seed=seed), seed + 1)
+    tok, _ = tokens_uniform(seed + 2, cfg.vocab, B, p0 + steps)
+    with hb.Context(cfg.to_rh(), 0, B, max_ctx or p0 + steps) as c:
+        c.load_weights(w.embed, w.gamma_final, [lw.tensors() for lw in w.layers])
+        want = c.forward(tok).logits
+        c.prefill(tok[:, :p0])
+        for p in range(p0, p0 + steps):
+            got = c.decode_step(tok[:, p], want_logits=True)[1]
+            assert np.abs(got - want[:, p]).max() <= LOGIT_ATOL, (B, p)
+
+
+# RMSNorm inside the decode GEMVs, a wave per token or the block for each:
+# rows shorter than a wave's 256 columns, ending inside and on one; fewer
+# tokens than waves, as many, more, and a ragged last round.
+@pytest.mark.parametrize("heads,B", [(2, 2), (2, 16), (6, 5), (10, 3), (10, 9), (16, 16), (42, 2), (42, 3), (42, 5)])
+def test_decode_norm_waves(heads, B):
+    cfg = small_cfg(dim=64 * heads, hidden=256, heads=heads, hd=64, nlayers=2, vocab=512, seq=24)
+    _decode_matches_forward(cfg, B, 5, 4, 310 + heads + B)
