@@ -756,11 +756,19 @@ hipError_t launch_attn_prefill(const f16* q, const f16* k, const f16* v, f16* ou
 
 // Small batches: chunks of ATTN_DEC_CHUNK positions over the whole cache
 // (ceil(ctx / ATTN_DEC_CHUNK) blocks per (head, sequence), those past the
-// current position exit at once).  Once B * H blocks fill the chip: one
-// chunk per (head, sequence).  Measured at 7B, ctx 2176: B 1 7.3 us +
-// 3.5 us merge (128-position chunks; 8 or 16 whole-context chunks took
-// 9.2 - 9.6 us), B 16 86 us (one chunk) vs 91 (128-position chunks).
+// current position exit at once).  Once B * H blocks fill the chip, or the
+// cache is short: one chunk per (head, sequence), which writes the output
+// itself.  Measured at 7B, ctx 2176: B 1 7.3 us + 3.5 us merge (128-position
+// chunks; 8 or 16 whole-context chunks took 9.2 - 9.6 us), B 16 86 us (one
+// chunk) vs 91 (128-position chunks).  The merge launch (about 5 us a layer)
+// buys its time back near 600 positions: whole generation passes with one
+// chunk against several, caches of 224 / 364 / 584 positions: 7B width, 1
+// sequence, 10.59 -> 10.33, 10.85 -> 10.73 and 11.20 -> 11.21 ms.
 int attn_decode_chunks(int B, int H, int ctx) {
+    return ctx <= 4 * ATTN_DEC_CHUNK ? 1 : attn_decode_chunks_max(B, H, ctx);
+}
+
+int attn_decode_chunks_max(int B, int H, int ctx) {
     return B * H >= 256 ? 1 : (ctx + ATTN_DEC_CHUNK - 1) / ATTN_DEC_CHUNK;
 }
 

@@ -120,6 +120,8 @@ hipError_t launch_attn_decode(const f16* q, const f16* k, const f16* v, const in
                               float* part_m, float* part_l, float* part_o, f16* out, int B, int H,
                               int hd, int ctx, hipStream_t st, int nch = 0, bool out_frag = false);
 int attn_decode_chunks(int B, int H, int ctx);
+// Chunks per (b, h) that the partials are sized for (>= attn_decode_chunks).
+int attn_decode_chunks_max(int B, int H, int ctx);
 
 // ---------------- decode GEMV (B <= 16 tokens) ----------------
 enum GemvEpi { GV_F32 = 0, GV_RESID = 1, GV_SWIGLU = 2, GV_QKV = 3 };

@@ -119,3 +119,13 @@ def _decode_matches_forward(cfg, B, p0, steps, seed, max_ctx=0):
 def test_decode_norm_waves(heads, B):
     cfg = small_cfg(dim=64 * heads, hidden=256, heads=heads, hd=64, nlayers=2, vocab=512, seq=24)
     _decode_matches_forward(cfg, B, 5, 4, 310 + heads + B)
+
+
+# Decode attention over one chunk (caches up to 512 positions) and several, at
+# the first and last positions of each.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("max_ctx,p0", [(129, 127), (512, 1), (512, 509), (513, 3), (513, 510)])
+def test_decode_attention_chunks(hd, max_ctx, p0):
+    cfg = small_cfg(dim=2 * hd if hd == 64 else hd, hidden=256, heads=2 if hd == 64 else 1, hd=hd, nlayers=2,
+                    vocab=512, seq=64)
+    _decode_matches_forward(cfg, 2, p0, min(3, max_ctx - p0), 330 + p0, max_ctx)
