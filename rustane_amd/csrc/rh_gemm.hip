@@ -623,6 +623,7 @@ __global__ __launch_bounds__(Tl::NT) void gemm_kernel(GemmArgs a, int P, long lo
         b.ldo = a.N;
         b.softcap = 0.f;
         b.alpha = 0.f;  // raw partials: the row kernel applies alpha once to their sum
+        b.part_cols = 0;
         run_epilogue<Tl, EPI_F32>(b, Tl::nw(nb * Tl::BN), Tl::mw(mb * Tl::BM), acc);
     } else {
         constexpr int NT = Tl::NT;
@@ -814,6 +815,34 @@ __global__ __launch_bounds__(Tl::NT + 64 * WG_SW) void gemm_wgrad_kernel(GemmArg
     }
 }
 
+// Data-parallel tiles: estimated time = rounds of one block per CU x
+// tile FLOPs / that tile's per-CU rate.  The rates are fitted to MI355X
+// timings of every tile on 27 GEMM shapes of the 7B forward and
+// training step (M 512 - 8192, random fp16 operands; the picks land
+// within 0.5% of the per-shape best in total; 256x256 and 256x128 refitted
+// for the ping-pong tiles: at M = 8192 a 256x256 tile takes 1.20 times a
+// 192x256 one's time for 1.33 times its work, at M = 512 1.09 times for a
+// tile of W1|W3); the estimate trades wave
+// quantization (e.g. 172 vs 230 tiles at M = 512) against per-tile
+// efficiency.  Narrow outputs (Wo) and long K (W2) use stream-K
+// instead, when every block gets at least two 32-wide k-iterations.  *cost: the
+// pick's estimate (per unit of K).
+int tile_pick(int M, int N, float* cost) {
+    struct Cand { int cfg, bn, bm; float rate; };
+    constexpr Cand dp[] = {{GCFG_D8_256x256, 256, 256, 5.0f}, {GCFG_D8_192x256, 192, 256, 4.35f},
+                           {GCFG_D8_256x128, 256, 128, 3.75f}, {GCFG_D8_192x128, 192, 128, 3.7f},
+                           {GCFG_D8_128x128, 128, 128, 3.0f}};
+    float best = 3.0e38f;
+    int cfg = 0;
+    for (const Cand& c : dp) {
+        const long long tiles = (long long)((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm);
+        const float t = (float)((tiles + SK_P - 1) / SK_P) * (float)c.bn * (float)c.bm / c.rate;
+        if (t < best) { best = t; cfg = c.cfg; }
+    }
+    if (cost) *cost = best;
+    return cfg;
+}
+
 using Tile256x256 = PTile<2, 4, 8, 4, 1, 4>;
 using Tile256x128 = PTile<4, 2, 4, 4, 2, 3>;
 
@@ -824,21 +853,6 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
         if (cfg == GCFG_AUTO && a.M <= SKINNY_M) return launch_gemm_skinny(EPI, a, st);
     }
     if (cfg == GCFG_AUTO) {
-        // Data-parallel tiles: estimated time = rounds of one block per CU x
-        // tile FLOPs / that tile's per-CU rate.  The rates are fitted to MI355X
-        // timings of every tile on 27 GEMM shapes of the 7B forward and
-        // training step (M 512 - 8192, random fp16 operands; the picks land
-        // within 0.5% of the per-shape best in total; 256x256 and 256x128 refitted
-        // for the ping-pong tiles: at M = 8192 a 256x256 tile takes 1.20 times a
-        // 192x256 one's time for 1.33 times its work, at M = 512 1.09 times for a
-        // tile of W1|W3); the estimate trades wave
-        // quantization (e.g. 172 vs 230 tiles at M = 512) against per-tile
-        // efficiency.  Narrow outputs (Wo) and long K (W2) use stream-K
-        // instead, when every block gets at least two 32-wide k-iterations.
-        struct Cand { int cfg, bn, bm; float rate; };
-        constexpr Cand dp[] = {{GCFG_D8_256x256, 256, 256, 5.0f}, {GCFG_D8_192x256, 192, 256, 4.35f},
-                               {GCFG_D8_256x128, 256, 128, 3.75f}, {GCFG_D8_192x128, 192, 128, 3.7f},
-                               {GCFG_D8_128x128, 128, 128, 3.0f}};
         const long long KT = a.K / 32;
         const int t256x128 = ((a.N + 255) / 256) * ((a.M + 127) / 128);
         const int t128 = ((a.N + 127) / 128) * ((a.M + 127) / 128);
@@ -852,12 +866,7 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
             // faster (15.3 + 8.5 us stream-K + fix-up against one 17.5 us round)
             cfg = GCFG_D8_128x128_SK;
         } else {
-            float best = 3.0e38f;
-            for (const Cand& c : dp) {
-                const long long tiles = (long long)((a.N + c.bn - 1) / c.bn) * ((a.M + c.bm - 1) / c.bm);
-                const float t = (float)((tiles + SK_P - 1) / SK_P) * (float)c.bn * (float)c.bm / c.rate;
-                if (t < best) { best = t; cfg = c.cfg; }
-            }
+            cfg = tile_pick(a.M, a.N, nullptr);
         }
     }
     // The 8-wave 192x256, 192x128 and 128x128 tiles run the 16x16x32 form: at
@@ -961,8 +970,18 @@ hipError_t launch_gemm_resid_norm(const GemmArgs& a, const float* gamma, float e
     return launch_rmsnorm(a.out_f32, gamma, xn, a.M, a.N, eps, st, true);
 }
 
+float gemm_tile_cost(int M, int N) {
+    float c = 0.f;
+    (void)tile_pick(M, N, &c);
+    return c;
+}
+
 hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t st) {
     if (a.K % 128 != 0 || a.N % 4 != 0 || a.M <= 0) return hipErrorInvalidValue;
+    if (a.part_cols && ((epi != EPI_F32 && epi != EPI_RESID) || a.part_cols % 4 != 0 || a.N > 3 * a.part_cols ||
+                        a.ldo != a.part_cols || a.resid_in || !a.out_part1 ||
+                        (a.N > 2 * a.part_cols && !a.out_part2)))
+        return hipErrorInvalidValue;
     switch (epi) {
         case EPI_F32: return launch_epi<EPI_F32>(a, st);
         case EPI_RESID: return launch_epi<EPI_RESID>(a, st);

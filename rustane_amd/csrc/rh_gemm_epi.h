@@ -26,6 +26,18 @@ __device__ __forceinline__ void silu_bwd4(const GemmArgs& a, int m, int n, float
     *(f16x4*)(a.out_f16 + frag_off(m, a.ldo + n, 2 * a.ldo)) = o3;
 }
 
+// The fp32 output that holds feature n; n becomes the feature's column in it.
+// (The pointers are read before the choice: a choice between fields would put
+// the argument copies of the split kernels in scratch memory.)
+__device__ __forceinline__ float* out_part(const GemmArgs& a, int& n) {
+    float *p0 = a.out_f32, *p1 = a.out_part1, *p2 = a.out_part2;
+    const int c = a.part_cols;
+    if (c == 0) return p0;
+    const int k = (n >= c) + (n >= 2 * c);
+    n -= k * c;
+    return k == 0 ? p0 : k == 1 ? p1 : p2;
+}
+
 // Stores four consecutive output features n..n+3 of token m (every epilogue
 // but SwiGLU, whose lanes hold W1 and W3 rows and store gate features).
 template <int EPI>
@@ -39,13 +51,14 @@ __device__ __forceinline__ void store4(const GemmArgs& a, int m, int n, float v0
             v0 = tanhf(v0 * ic) * c; v1 = tanhf(v1 * ic) * c;
             v2 = tanhf(v2 * ic) * c; v3 = tanhf(v3 * ic) * c;
         }
-        f32x4* po = (f32x4*)(a.out_f32 + (size_t)m * a.ldo + n);
+        f32x4* po = (f32x4*)(out_part(a, n) + (size_t)m * a.ldo + n);
         if (a.nt_out) __builtin_nontemporal_store(f32x4{v0, v1, v2, v3}, po);
         else *po = f32x4{v0, v1, v2, v3};
     } else if constexpr (EPI == EPI_RESID) {
+        float* out = out_part(a, n);
         const size_t o = (size_t)m * a.ldo + n;
-        f32x4* px = (f32x4*)(a.out_f32 + o);
-        f32x4 x = *(const f32x4*)((a.resid_in ? a.resid_in : a.out_f32) + o);
+        f32x4* px = (f32x4*)(out + o);
+        f32x4 x = *(const f32x4*)((a.resid_in ? a.resid_in : out) + o);
         x[0] = v0 * a.alpha + x[0]; x[1] = v1 * a.alpha + x[1];
         x[2] = v2 * a.alpha + x[2]; x[3] = v3 * a.alpha + x[3];
         if (a.nt_out) __builtin_nontemporal_store(x, px);

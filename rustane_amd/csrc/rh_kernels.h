@@ -37,6 +37,10 @@ struct GemmArgs {
     size_t sk_part_floats;
     int force_cfg;  // 0 = heuristic; otherwise a GemmCfg value (tuning)
     bool nt_out;    // EPI_F32 / EPI_RESID: nontemporal output stores (data read much later)
+    // EPI_F32 / EPI_RESID (in place): part_cols > 0 cuts the N features into up
+    // to three outputs [M][ldo = part_cols]: out_f32, out_part1, out_part2.
+    int part_cols;
+    float *out_part1, *out_part2;
     // Optional timing: stamped at the kernel's own start and end by the
     // one-block-per-tile launch (hipExtLaunchKernelGGL), recorded around the
     // launches otherwise.
@@ -77,6 +81,8 @@ constexpr int SKINNY_M = 64;
 int skinny_splits(const GemmArgs& a);
 hipError_t launch_gemm_skinny(int epi, const GemmArgs& a, hipStream_t st);
 hipError_t launch_gemm_skinny_split(const GemmArgs& a, int S, hipStream_t st);
+// The tile model's estimate for an [M][N] output, per unit of K.
+float gemm_tile_cost(int M, int N);
 // Floats of stream-K workspace any prefill GEMM needs.
 size_t gemm_sk_part_floats();
 hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t st);

@@ -115,6 +115,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(GemmArgs a, int S) {
         b.ldo = a.N;
         b.softcap = 0.f;
         b.alpha = 0.f;  // raw partials: the row kernel applies alpha once to their sum
+        b.part_cols = 0;
     }
     constexpr int PT = EPI == EPI_SWIGLU ? 2 : 1;  // row tiles stored together (W1 rows and the matching W3 rows)
     for (int x = w; x < RT / PT * MT; x += NW) {

@@ -322,36 +322,45 @@ int gamma_grad(rh_ctx* ctx, int nblk, int D, float kappa, float* dgamma) {
 
 // C[rows][cols] += kappa * X W^T with X [rows][Mp], W [cols][Mp] (token-inner).
 // When every gradient is still zero the epilogue stores kappa * acc instead
-// (the same values; it skips reading the fp32 gradient back).  K is the
-// token count, short next to the fp32 output these GEMMs write, so the tile
-// is picked from MI355X timings at K = 512 / 2048 / 8192 (store | accumulate
-// epilogue, us) rather than by the FLOP model:
-//   4096 x 4096:  256x128 8-wave 29.6 | 39.1, 73.7 | 79.1  (192x128 4-wave
-//                 34 | 55, 84 | 97); at K 8192 the model's pick, 280 | 297
-//   4096 x 11008: 192x256 8-wave 80 | 105, 220 | 242, 744 | 790  (192x128
-//                 4-wave 88 | 124, 263 | 278)
-//   32000 x 4096 (tied embedding): 192x256 256 | 364, 694 | 772; at K 8192
-//                 256x128 2079 | 2164
-// On the side stream (st != the context's stream) no stream-K: its workspace
-// belongs to the main stream's GEMMs.
+// (the same values; it skips reading the fp32 gradient back).  The tile model
+// picks the tile (no stream-K: its workspace belongs to the main stream's
+// GEMMs); its picks at K = 4096, accumulating, against the best of the other
+// tiles (us): 4096 x 4096 256x256 112 | 122, 4096 x 11008 256x256 355 | 394,
+// 8192 x 4096 256x256 223 | 252; 1024 x 1024 128x128 28 | 39, 1024 x 2816
+// 128x128 31 | 40, 8192 x 1024 256x128 62 | 68.  A short K after a zero leaves
+// the fp32 output most of the time; large outputs then take the kernel whose
+// store waves write a tile while the next one is computed.
 int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* out,
               hipStream_t st) {
     rh::GemmArgs g{};
     g.X = X; g.W = W; g.M = rows; g.N = cols; g.K = ctx->train->Mp;
     g.out_f32 = out; g.ldo = cols; g.alpha = kappa;
     g.nt_out = true;  // read only by the optimizer
-    const bool long_k = g.K >= 8192;
     if (ctx->train->zero && g.K <= 1024 && (size_t)rows * cols >= (size_t)4096 * 4096) {
         LCK(rh::launch_gemm_wgrad(g, false, st));
         return RH_OK;
     }
-    if (cols > 4096)
-        g.force_cfg = rh::GCFG_D8_192x256;
-    else if (rows > 4096)
-        g.force_cfg = long_k ? rh::GCFG_D8_256x128 : rh::GCFG_D8_192x256;
-    else
-        g.force_cfg = long_k ? rh::GCFG_AUTO : rh::GCFG_D8_256x128;
-    if (st == ctx->stream) set_sk(ctx, g);
+    LCK(rh::launch_gemm(ctx->train->zero ? rh::EPI_F32 : rh::EPI_RESID, g, st));
+    return RH_OK;
+}
+
+// n (2 or 3) gradients [rows][cols] of one X, the W of each after the other:
+// dWq | dWk | dWv and dW1 | dW3.  As one product with n outputs where that
+// fills the CUs better than n products (the tile model's estimate): 1024 wide
+// at K = 4096, dWq..dWv 85 -> 32 us, dW1 dW3 62 -> 50; 4096 wide three products
+// of one round each stay (334 against 358 us).
+int grad_gemms(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* const* out, int n,
+               hipStream_t st) {
+    if (rh::gemm_tile_cost(rows, n * cols) >= (float)n * rh::gemm_tile_cost(rows, cols)) {
+        for (int j = 0; j < n; ++j)
+            RCK(grad_gemm(ctx, X, W + (size_t)j * cols * ctx->train->Mp, rows, cols, kappa, out[j], st));
+        return RH_OK;
+    }
+    rh::GemmArgs g{};
+    g.X = X; g.W = W; g.M = rows; g.N = n * cols; g.K = ctx->train->Mp;
+    g.out_f32 = out[0]; g.out_part1 = out[1]; g.out_part2 = n > 2 ? out[2] : nullptr;
+    g.part_cols = g.ldo = cols; g.alpha = kappa;
+    g.nt_out = true;
     LCK(rh::launch_gemm(ctx->train->zero ? rh::EPI_F32 : rh::EPI_RESID, g, st));
     return RH_OK;
 }
@@ -442,8 +451,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         RCK(publish(1));
         LCK(rh::launch_transpose_frag2(T->H2, X1[0], M, 2 * F, cc.x2n, X1[1], M, D, Mp, sd));
         HCK(hipEventRecord(T->read[1], sd));
-        RCK(grad_gemm(ctx, X1[1], X1[0], D, F, kappa, G[4], sd));
-        RCK(grad_gemm(ctx, X1[1], X1[0] + (size_t)F * Mp, D, F, kappa, G[5], sd));
+        RCK(grad_gemms(ctx, X1[1], X1[0], D, F, kappa, G + 4, 2, sd));
         RCK(data_gemm(ctx, T->H2, wt.w13t, M, D, 2 * F, T->gout, &dp, &ns));
         // dx2 = RMSNorm2'(dx_ffn) + dy (in place in dres); a*dx2 -> H1m
         RCK(rewrite(2));
@@ -465,8 +473,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         RCK(publish(3));
         LCK(rh::launch_transpose_frag2(T->H2q, X3[0], M, 3 * D, cc.xn, X3[1], M, D, Mp, sd));
         HCK(hipEventRecord(T->read[3], sd));
-        for (int j = 0; j < 3; ++j)
-            RCK(grad_gemm(ctx, X3[1], X3[0] + (size_t)j * D * Mp, D, D, kappa, G[j], sd));
+        RCK(grad_gemms(ctx, X3[1], X3[0], D, D, kappa, G, 3, sd));
         RCK(data_gemm(ctx, T->H2q, wt.qkvt, M, D, 3 * D, T->gout, &dp, &ns));
         // dy' = RMSNorm1'(dxn) + dx2 (in place); a*dy' -> H1 (the next layer's dffn)
         RCK(rewrite(0));

@@ -129,3 +129,14 @@ def test_decode_attention_chunks(hd, max_ctx, p0):
     cfg = small_cfg(dim=2 * hd if hd == 64 else hd, hidden=256, heads=2 if hd == 64 else 1, hd=hd, nlayers=2,
                     vocab=512, seq=64)
     _decode_matches_forward(cfg, 2, p0, min(3, max_ctx - p0), 330 + p0, max_ctx)
+
+
+# Weight gradients of one input as one product with two or three outputs
+# (narrow models): tiles that straddle the outputs, stored and accumulated.
+@pytest.mark.parametrize("heads,hidden", [(1, 128), (3, 640), (5, 1408)])
+@pytest.mark.parametrize("calls", [1, 2])
+def test_joint_weight_gradients(orc, heads, hidden, calls):
+    cfg = small_cfg(dim=128 * heads, hidden=hidden, heads=heads, hd=128, nlayers=1, vocab=512, seq=70)
+    w = random_gammas(ModelWeights.normal(cfg, seed=340 + heads, std=0.05), 341)
+    tok, tgt = tokens_uniform(342, cfg.vocab, 2, cfg.seq)
+    _run(orc, cfg, w, tok, tgt, calls=calls)
