@@ -251,37 +251,54 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_kernel(const f16* __restric
     }
 }
 
-// hd 128: the same two kernels with their operand tiles moved global -> LDS
-// by DMA (global_load_lds_dwordx4, 16 bytes per lane at LDS base + 16 lane)
-// through a two-stage pipeline, so the next tile's loads are in flight while
-// this one is computed and no VGPRs or LDS stores stage them.  Tiles keep
-// their natural [row][hd] order (256-byte rows) with the XOR chunk swizzles
-// of the forward kernel: a tile read as row fragments (an A operand with
-// rows = keys or queries) is stored with swz_k, one read transposed (K^T,
-// Q^T, dO^T) with swz_v and read by ds_read_b64_tr_b16, so K (dq) and Q, dO
-// (dk/dv) are moved twice, once per swizzle.  The MFMA operands and their
-// order are those of the kernels above, so the results are identical.
+// hd 128: the same two kernels as the two halves of one launch, with their
+// operand tiles moved global -> LDS by DMA (global_load_lds_dwordx4, 16 bytes
+// per lane at LDS base + 16 lane) through a two-stage pipeline, so the next
+// tile's loads are in flight while this one is computed and no VGPRs or LDS
+// stores stage them.  Tiles keep their natural [row][hd] order (256-byte rows)
+// with an XOR chunk swizzle (swz_b) under which both the row-fragment reads
+// and the transposing reads (ds_read_b64_tr_b16: K^T, Q^T, dO^T) are free of
+// bank conflicts, so one copy of a tile serves both.  The MFMA operands and
+// their order are those of the kernels above, so the results are identical.
+//
+// What bounds it: a block is 4 waves, one per SIMD, in a chain of LDS reads,
+// MFMAs, exp2 and a barrier, so a lone block leaves every unit idle most of the
+// time.  A copy per kind of read (96 and 128 KB of LDS, one block per CU) ran
+// at 134 TFLOP/s; 64 KB lets two blocks share a CU, and one launch for both
+// halves fills the first half's last wave with the second's blocks.
+// Measured alone (dQ + dK/dV, us): 8 sequences x 8 heads x 512 92 -> 50, 8 x 32 x
+// 512 321 -> 168 (256 TFLOP/s; LDS reads alone would take about 60).
 //
 // Wave w moves 1 KB units w, w + 4, w + 8, w + 12 of a 64-row tile (unit i
 // holds rows 4i..4i+3; lane L row 4i + L/16 and stored chunk L%16).
-__device__ __forceinline__ void dma_tile(const f16* __restrict__ base, int r0, int S, f16* dst, bool tr) {
+constexpr int BWD_HD = 128, BWD_RB = 64, BWD_TILE = BWD_RB * BWD_HD;
+
+// Chunk c of row k is stored at c ^ swz_b(k).  Row-fragment reads (16 lanes:
+// rows 8(r/4) + 4u + r%4, one chunk) see 16 different values of row bits 0, 1,
+// 3, 4, hence 16 different chunks; transposing reads (16 lanes: rows 8g + 4h +
+// r/4, chunks 2j and 2j + 1) see row bits 0, 1 in chunk bits 1, 2 and the chunk
+// pair in bit 0, hence 8 different chunks, and 16 over lane groups g, g + 1.
+__device__ __forceinline__ int swz_b(int row) {
+    return ((row & 3) << 1) | (((row >> 3) & 1) << 3) | ((row >> 4) & 1);
+}
+
+__device__ __forceinline__ void dma_tile(const f16* __restrict__ base, int r0, int S, f16* dst) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
         const int i = w + 4 * t, row = 4 * i + (lane >> 4);
-        const int sw = tr ? swz_v(row) : swz_k(row);
-        const f16* src = base + (size_t)min(r0 + row, S - 1) * 128 + 8 * ((lane & 15) ^ sw);
+        const f16* src = base + (size_t)min(r0 + row, S - 1) * BWD_HD + 8 * ((lane & 15) ^ swz_b(row));
         __builtin_amdgcn_global_load_lds((const void*)src, (__attribute__((address_space(3))) void*)(dst + i * 512),
                                          16, 0, 0);
     }
 }
 
-// Row fragment of a swz_k tile: 8 hd values 32kk + 8g .. +7 of row `row`.
+// Row fragment of a tile: 8 hd values 32kk + 8g .. +7 of row `row`.
 __device__ __forceinline__ f16x8 tile_row(const f16* t, int row, int kk, int g) {
-    return *(const f16x8*)&t[row * 128 + 8 * ((4 * kk + g) ^ swz_k(row))];
+    return *(const f16x8*)&t[row * BWD_HD + 8 * ((4 * kk + g) ^ swz_b(row))];
 }
 
-// Transposed fragment of a swz_v tile: element e = T[32c + 8g + e][16j + r]
+// Transposed fragment of a tile: element e = T[32c + 8g + e][16j + r]
 // (rows of the tile as the k dimension), from two transposing reads.
 __device__ __forceinline__ f16x8 tile_tr(const f16* t, int c, int j, int lane) {
     const int g = (lane >> 4) & 3, r = lane & 15, ch = 2 * j + ((lane & 3) >> 1);
@@ -289,7 +306,7 @@ __device__ __forceinline__ f16x8 tile_tr(const f16* t, int c, int j, int lane) {
 #pragma unroll
     for (int hh = 0; hh < 2; ++hh) {
         const int row = 32 * c + 8 * g + 4 * hh + (r >> 2);
-        const f16* a = &t[row * 128 + 8 * (ch ^ swz_v(row)) + 4 * (lane & 1)];
+        const f16* a = &t[row * BWD_HD + 8 * (ch ^ swz_b(row)) + 4 * (lane & 1)];
         const f16x4 v = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                                                       (__attribute__((address_space(3))) s16x4*)a));
 #pragma unroll
@@ -298,43 +315,47 @@ __device__ __forceinline__ f16x8 tile_tr(const f16* t, int c, int j, int lane) {
     return out;
 }
 
-__global__ __launch_bounds__(256) void attn_bwd_dq_dma_kernel(const f16* __restrict__ Q, const f16* __restrict__ K,
-                                                              const f16* __restrict__ V, const f16* __restrict__ dO,
-                                                              const float* __restrict__ lse,
-                                                              const float* __restrict__ Drow,
-                                                              f16* __restrict__ dqkv, const float2* __restrict__ rope,
-                                                              int H, int S, float scale_log2, float scale) {
-    constexpr int HD = 128, KB = 64, NKK = HD / 32, NHT = HD / 16, TILE = KB * HD;
-    // one array per stage and role, so the compiler's wait-count tracking
-    // tells a stage's reads from the DMA filling the other stage
-    __shared__ __attribute__((aligned(1024))) f16 sK0[TILE], sV0[TILE], sKt0[TILE], sK1[TILE], sV1[TILE],
-        sKt1[TILE];
+struct AttnBwdArgs {
+    const f16 *Q, *K, *V, *dO;
+    const float *lse, *Drow;
+    f16* dqkv;
+    const float2* rope;
+    int H, S;
+    float scale_log2, scale;
+};
+
+// dQ of one tile of 64 queries (the block's tile t of all B * H * ceil(S / 64)).
+// x0, y0 and x1, y1 are the two stages' tiles; one array per stage and role, so
+// the compiler's wait-count tracking tells a stage's reads from the DMA filling
+// the other stage.
+__device__ __forceinline__ void attn_bwd_dq_dma(const AttnBwdArgs& a, int t, f16* x0, f16* y0, f16* x1, f16* y1) {
+    constexpr int HD = BWD_HD, KB = BWD_RB, NKK = HD / 32, NHT = HD / 16;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, r = lane & 15;
+    const int S = a.S, H = a.H;
     const int nqt = (S + 63) / 64;
-    const int t = xcd_remap((int)blockIdx.x, (int)gridDim.x);
     const int qt = nqt - 1 - t % nqt;  // longest rows first
     const int h = (t / nqt) % H, b = t / nqt / H;
     const int q0 = qt * 64, qi = q0 + w * 16 + r, qrow = min(qi, S - 1);
     const size_t bh = (size_t)b * H + h;
-    const f16* Kb = K + bh * S * HD;
-    const f16* Vb = V + bh * S * HD;
-    f16x8 qf[NKK], df[NKK];
-#pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) {
-        qf[kk] = *(const f16x8*)(Q + (bh * S + qrow) * HD + 32 * kk + 8 * g);
-        df[kk] = *(const f16x8*)(dO + (bh * S + qrow) * HD + 32 * kk + 8 * g);
-    }
-    const float L = lse[bh * S + qrow], Dq = Drow[bh * S + qrow];
-    f32x4 acc[NHT];
-#pragma unroll
-    for (int j = 0; j < NHT; ++j) acc[j] = f32x4{};
+    const f16* Kb = a.K + bh * S * HD;
+    const f16* Vb = a.V + bh * S * HD;
     const int nkb = (min(S, q0 + 64) + KB - 1) / KB;
     auto issue = [&](int kb, auto ST) {
         constexpr int st = decltype(ST)::value;
-        dma_tile(Kb, kb * KB, S, st ? sK1 : sK0, false);
-        dma_tile(Vb, kb * KB, S, st ? sV1 : sV0, false);
-        dma_tile(Kb, kb * KB, S, st ? sKt1 : sKt0, true);
+        dma_tile(Kb, kb * KB, S, st ? x1 : x0);
+        dma_tile(Vb, kb * KB, S, st ? y1 : y0);
     };
+    issue(0, std::integral_constant<int, 0>{});
+    f16x8 qf[NKK], df[NKK];
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+        qf[kk] = *(const f16x8*)(a.Q + (bh * S + qrow) * HD + 32 * kk + 8 * g);
+        df[kk] = *(const f16x8*)(a.dO + (bh * S + qrow) * HD + 32 * kk + 8 * g);
+    }
+    const float L = a.lse[bh * S + qrow], Dq = a.Drow[bh * S + qrow];
+    f32x4 acc[NHT];
+#pragma unroll
+    for (int j = 0; j < NHT; ++j) acc[j] = f32x4{};
     auto step = [&](int kb, auto ST) {
         constexpr int cur = decltype(ST)::value;
         const int k0 = kb * KB;
@@ -344,9 +365,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_dma_kernel(const f16* __restr
         wait_vm<0>();
         lds_barrier();
         if (kb + 1 < nkb) issue(kb + 1, std::integral_constant<int, 1 - cur>{});
-        const f16* sK = cur ? sK1 : sK0;
-        const f16* sV = cur ? sV1 : sV0;
-        const f16* sKt = cur ? sKt1 : sKt0;
+        const f16* sK = cur ? x1 : x0;
+        const f16* sV = cur ? y1 : y0;
         f32x4 sc[2][2], dp[2][2];
 #pragma unroll
         for (int c = 0; c < 2; ++c)
@@ -370,15 +390,15 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_dma_kernel(const f16* __restr
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const bool live = 32 * c + 4 * u + i <= lim;
-                    const float p = live ? __builtin_amdgcn_exp2f(__builtin_fmaf(sc[c][u][i], scale_log2, -L)) : 0.f;
+                    const float p =
+                        live ? __builtin_amdgcn_exp2f(__builtin_fmaf(sc[c][u][i], a.scale_log2, -L)) : 0.f;
                     dsf[c][4 * u + i] = (f16)(p * (dp[c][u][i] - Dq));
                 }
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-            for (int j = 0; j < NHT; ++j) acc[j] = mfma16(tile_tr(sKt, c, j, lane), dsf[c], acc[j]);
+            for (int j = 0; j < NHT; ++j) acc[j] = mfma16(tile_tr(sK, c, j, lane), dsf[c], acc[j]);
     };
-    issue(0, std::integral_constant<int, 0>{});
     for (int kb0 = 0; kb0 < nkb; kb0 += 2) {
         step(kb0, std::integral_constant<int, 0>{});
         if (kb0 + 1 < nkb) step(kb0 + 1, std::integral_constant<int, 1>{});
@@ -386,69 +406,57 @@ __global__ __launch_bounds__(256) void attn_bwd_dq_dma_kernel(const f16* __restr
     if (qi < S) {
 #pragma unroll
         for (int j = 0; j < NHT; ++j)
-            store_dqkv4<HD>(dqkv, rope, b * S + qi, qi, 0, H * HD, h, 16 * j + 4 * g, acc[j] * scale);
+            store_dqkv4<HD>(a.dqkv, a.rope, b * S + qi, qi, 0, H * HD, h, 16 * j + 4 * g, acc[j] * a.scale);
     }
 }
 
-__global__ __launch_bounds__(256) void attn_bwd_dkdv_dma_kernel(const f16* __restrict__ Q,
-                                                                const f16* __restrict__ K,
-                                                                const f16* __restrict__ V,
-                                                                const f16* __restrict__ dO,
-                                                                const float* __restrict__ lse,
-                                                                const float* __restrict__ Drow,
-                                                                f16* __restrict__ dqkv, const float2* __restrict__ rope,
-                                                            int H, int S,
-                                                                float scale_log2, float scale) {
-    constexpr int HD = 128, QB = 64, NKK = HD / 32, NHT = HD / 16, TILE = QB * HD;
-    __shared__ __attribute__((aligned(1024))) f16 sQ0[TILE], sO0[TILE], sQt0[TILE], sOt0[TILE], sQ1[TILE],
-        sO1[TILE], sQt1[TILE], sOt1[TILE];
-    __shared__ __attribute__((aligned(256))) float sL0[QB], sD0[QB], sL1[QB], sD1[QB];
+// dK and dV of one tile of 64 keys; l0, d0 and l1, d1: the stages' lse and D.
+__device__ __forceinline__ void attn_bwd_dkdv_dma(const AttnBwdArgs& a, int t, f16* x0, f16* y0, f16* x1, f16* y1,
+                                                  float* l0, float* d0, float* l1, float* d1) {
+    constexpr int HD = BWD_HD, QB = BWD_RB, NKK = HD / 32, NHT = HD / 16;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, r = lane & 15;
+    const int S = a.S, H = a.H;
     const int nkt = (S + 63) / 64;
-    const int t = xcd_remap((int)blockIdx.x, (int)gridDim.x);  // a head's tiles share an XCD's L2
     const int kt = t % nkt;  // the first key blocks see the most queries: launched first
     const int h = (t / nkt) % H, b = t / nkt / H;
     const int k0 = kt * 64, ki = k0 + w * 16 + r, krow = min(ki, S - 1);
     const size_t bh = (size_t)b * H + h;
-    const f16* Qb = Q + bh * S * HD;
-    const f16* dOb = dO + bh * S * HD;
-    f16x8 kf[NKK], vf[NKK];
-#pragma unroll
-    for (int kk = 0; kk < NKK; ++kk) {
-        kf[kk] = *(const f16x8*)(K + (bh * S + krow) * HD + 32 * kk + 8 * g);
-        vf[kk] = *(const f16x8*)(V + (bh * S + krow) * HD + 32 * kk + 8 * g);
-    }
-    f32x4 dk[NHT], dv[NHT];
-#pragma unroll
-    for (int j = 0; j < NHT; ++j) dk[j] = dv[j] = f32x4{};
+    const f16* Qb = a.Q + bh * S * HD;
+    const f16* dOb = a.dO + bh * S * HD;
     const int nqb = (S + QB - 1) / QB;
     auto issue = [&](int qb, auto ST) {
         constexpr int st = decltype(ST)::value;
         const int q0 = qb * QB;
-        dma_tile(Qb, q0, S, st ? sQ1 : sQ0, false);
-        dma_tile(dOb, q0, S, st ? sO1 : sO0, false);
-        dma_tile(Qb, q0, S, st ? sQt1 : sQt0, true);
-        dma_tile(dOb, q0, S, st ? sOt1 : sOt0, true);
+        dma_tile(Qb, q0, S, st ? x1 : x0);
+        dma_tile(dOb, q0, S, st ? y1 : y0);
         // the 64 queries' lse and D, 4 bytes per lane (every wave writes the
         // same values, so each wave's DMA count stays the same)
         const size_t qv = bh * S + min(q0 + lane, S - 1);
-        __builtin_amdgcn_global_load_lds((const void*)(lse + qv), (__attribute__((address_space(3))) void*)(st ? sL1 : sL0),
-                                         4, 0, 0);
-        __builtin_amdgcn_global_load_lds((const void*)(Drow + qv), (__attribute__((address_space(3))) void*)(st ? sD1 : sD0),
-                                         4, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(a.lse + qv),
+                                         (__attribute__((address_space(3))) void*)(st ? l1 : l0), 4, 0, 0);
+        __builtin_amdgcn_global_load_lds((const void*)(a.Drow + qv),
+                                         (__attribute__((address_space(3))) void*)(st ? d1 : d0), 4, 0, 0);
     };
+    issue(kt, std::integral_constant<int, 0>{});
+    f16x8 kf[NKK], vf[NKK];
+#pragma unroll
+    for (int kk = 0; kk < NKK; ++kk) {
+        kf[kk] = *(const f16x8*)(a.K + (bh * S + krow) * HD + 32 * kk + 8 * g);
+        vf[kk] = *(const f16x8*)(a.V + (bh * S + krow) * HD + 32 * kk + 8 * g);
+    }
+    f32x4 dk[NHT], dv[NHT];
+#pragma unroll
+    for (int j = 0; j < NHT; ++j) dk[j] = dv[j] = f32x4{};
     auto step = [&](int qb, auto ST) {
         constexpr int cur = decltype(ST)::value;
         const int q0 = qb * QB;
         wait_vm<0>();
         lds_barrier();
         if (qb + 1 < nqb) issue(qb + 1, std::integral_constant<int, 1 - cur>{});
-        const f16* sQ = cur ? sQ1 : sQ0;
-        const f16* sO = cur ? sO1 : sO0;
-        const f16* sQt = cur ? sQt1 : sQt0;
-        const f16* sOt = cur ? sOt1 : sOt0;
-        const float* sL = cur ? sL1 : sL0;
-        const float* sD = cur ? sD1 : sD0;
+        const f16* sQ = cur ? x1 : x0;
+        const f16* sO = cur ? y1 : y0;
+        const float* sL = cur ? l1 : l0;
+        const float* sD = cur ? d1 : d0;
         f32x4 s[2][2], dp[2][2];
 #pragma unroll
         for (int c = 0; c < 2; ++c)
@@ -472,7 +480,8 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_dma_kernel(const f16* __res
                 for (int i = 0; i < 4; ++i) {
                     const int qo = 32 * c + 8 * g + 4 * u + i, q = q0 + qo;
                     const bool live = q >= ki && q < S;
-                    const float p = live ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][u][i], scale_log2, -sL[qo])) : 0.f;
+                    const float p =
+                        live ? __builtin_amdgcn_exp2f(__builtin_fmaf(s[c][u][i], a.scale_log2, -sL[qo])) : 0.f;
                     pf[c][4 * u + i] = (f16)p;
                     dsf[c][4 * u + i] = (f16)(p * (dp[c][u][i] - sD[qo]));
                 }
@@ -480,11 +489,10 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_dma_kernel(const f16* __res
         for (int c = 0; c < 2; ++c)
 #pragma unroll
             for (int j = 0; j < NHT; ++j) {
-                dv[j] = mfma16(tile_tr(sOt, c, j, lane), pf[c], dv[j]);
-                dk[j] = mfma16(tile_tr(sQt, c, j, lane), dsf[c], dk[j]);
+                dv[j] = mfma16(tile_tr(sO, c, j, lane), pf[c], dv[j]);
+                dk[j] = mfma16(tile_tr(sQ, c, j, lane), dsf[c], dk[j]);
             }
     };
-    issue(kt, std::integral_constant<int, 0>{});
     for (int qb0 = kt; qb0 < nqb; qb0 += 2) {
         step(qb0, std::integral_constant<int, 0>{});
         if (qb0 + 1 < nqb) step(qb0 + 1, std::integral_constant<int, 1>{});
@@ -493,10 +501,22 @@ __global__ __launch_bounds__(256) void attn_bwd_dkdv_dma_kernel(const f16* __res
         const int D = H * HD;
 #pragma unroll
         for (int j = 0; j < NHT; ++j) {
-            store_dqkv4<HD>(dqkv, rope, b * S + ki, ki, 1, D, h, 16 * j + 4 * g, dk[j] * scale);
-            store_dqkv4<HD>(dqkv, rope, b * S + ki, ki, 2, D, h, 16 * j + 4 * g, dv[j]);
+            store_dqkv4<HD>(a.dqkv, a.rope, b * S + ki, ki, 1, D, h, 16 * j + 4 * g, dk[j] * a.scale);
+            store_dqkv4<HD>(a.dqkv, a.rope, b * S + ki, ki, 2, D, h, 16 * j + 4 * g, dv[j]);
         }
     }
+}
+
+// Blocks 0 .. n - 1 own the key tiles (the longer work), n .. 2n - 1 the query
+// tiles; a head's tiles share an XCD's L2 (xcd_remap).
+__global__ __launch_bounds__(256, 2) void attn_bwd_dma_kernel(AttnBwdArgs a, int n) {
+    __shared__ __attribute__((aligned(1024))) f16 x0[BWD_TILE], y0[BWD_TILE], x1[BWD_TILE], y1[BWD_TILE];
+    __shared__ __attribute__((aligned(256))) float l0[BWD_RB], d0[BWD_RB], l1[BWD_RB], d1[BWD_RB];
+    const int bid = (int)blockIdx.x;
+    if (bid < n)
+        attn_bwd_dkdv_dma(a, xcd_remap(bid, n), x0, y0, x1, y1, l0, d0, l1, d1);
+    else
+        attn_bwd_dq_dma(a, xcd_remap(bid - n, n), x0, y0, x1, y1);
 }
 
 // dO [M, H*hd] fp32 (token-major GEMM output, the sum of NS split-K
@@ -574,10 +594,8 @@ hipError_t launch_attn_backward(const f16* q, const f16* k, const f16* v, const 
     const dim3 grid((S + 63) / 64 * H * B);
     const float scale = 1.0f / sqrtf((float)hd), sl2 = scale * 1.4426950408889634f;
     if (hd == 128) {
-        hipLaunchKernelGGL(attn_bwd_dq_dma_kernel, grid, dim3(256), 0, st, q, k, v, dOh, lse, Drow, dqkv, rope, H, S, sl2,
-                           scale);
-        hipLaunchKernelGGL(attn_bwd_dkdv_dma_kernel, grid, dim3(256), 0, st, q, k, v, dOh, lse, Drow, dqkv, rope, H, S,
-                           sl2, scale);
+        const AttnBwdArgs a{q, k, v, dOh, lse, Drow, dqkv, rope, H, S, sl2, scale};
+        hipLaunchKernelGGL(attn_bwd_dma_kernel, dim3(2 * grid.x), dim3(256), 0, st, a, (int)grid.x);
     } else {
         hipLaunchKernelGGL((attn_bwd_dq_kernel<64>), grid, dim3(256), 0, st, q, k, v, dOh, lse, Drow, dqkv, rope, H, S,
                            sl2, scale);

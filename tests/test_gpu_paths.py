@@ -140,3 +140,14 @@ def test_joint_weight_gradients(orc, heads, hidden, calls):
     w = random_gammas(ModelWeights.normal(cfg, seed=340 + heads, std=0.05), 341)
     tok, tgt = tokens_uniform(342, cfg.vocab, 2, cfg.seq)
     _run(orc, cfg, w, tok, tgt, calls=calls)
+
+
+# Attention backward at head dim 128: lengths that end inside and on a 64-row
+# tile, and one, two and several tiles (both stages and the odd last one); six
+# heads' tiles do not share out evenly over the XCDs.
+@pytest.mark.parametrize("seq", [2, 63, 64, 65, 130, 320])
+def test_attention_backward_lengths(orc, seq):
+    cfg = small_cfg(dim=384, hidden=256, heads=3, hd=128, nlayers=1, vocab=512, seq=seq)
+    w = random_gammas(ModelWeights.normal(cfg, seed=350, std=0.05), 351)
+    tok, tgt = tokens_uniform(352 + seq, cfg.vocab, 2, cfg.seq)
+    _run(orc, cfg, w, tok, tgt)
