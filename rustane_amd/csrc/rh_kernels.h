@@ -233,9 +233,9 @@ hipError_t launch_transpose_frag2(const f16* src0, f16* dst0, int R0, int C0, co
                                   int C1, int Rp, hipStream_t st);
 // RMSNorm backward over M rows: dx = rmsnorm'(x)^T dy (+ dres), optional
 // fp16 fragment-order copy of hscale * dx, per-block dgamma partials
-// [rms_backward_blocks(M)][D].  dy is the sum of nsplit (1..8) fp32 partials
+// [rms_backward_blocks(M, D)][D].  dy is the sum of nsplit (1..8) fp32 partials
 // [M][D] split_stride floats apart, added in order.  dx may alias dres.
-int rms_backward_blocks(int M);
+int rms_backward_blocks(int M, int D);
 hipError_t launch_rms_backward(const float* dy, int nsplit, size_t split_stride, const float* x,
                                const float* gamma, const float* dres, float* dx, f16* outh, float hscale,
                                float* dg_part, int M, int D, float eps, hipStream_t st);

@@ -233,7 +233,7 @@ int ensure_train_ws(rh_ctx* ctx, int B, int S) {
     RCK(dalloc(ctx, &T->gout, m * D));  // an unsplit data-gradient product [M][D]
     RCK(dalloc(ctx, &T->dres, m * D));
     RCK(dalloc(ctx, &T->Drow, (size_t)M * c.heads));
-    RCK(dalloc(ctx, &T->dgp, (size_t)rh::rms_backward_blocks(M) * D));
+    RCK(dalloc(ctx, &T->dgp, (size_t)rh::rms_backward_blocks(M, (int)D) * D));
     RCK(dalloc(ctx, &T->utok, m));
     RCK(dalloc(ctx, &T->ustart, m + 1));
     RCK(dalloc(ctx, &T->uidx, m));
@@ -393,7 +393,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
     const int H = c.heads, hd = c.head_dim;
     const float alpha = 1.0f / std::sqrt(2.0f * (float)c.nlayers);
     const float kappa = loss_scale / ((float)S * rh::GRAD_UNIT);
-    const int nblk = rh::rms_backward_blocks(M);
+    const int nblk = rh::rms_backward_blocks(M, D);
     hipStream_t st = ctx->stream;
     // Main stream: the chain through the data gradients.  Side stream: the
     // weight gradients, each group from its own copies, after the activation

@@ -128,29 +128,36 @@ __global__ __launch_bounds__(256) void transpose_frag_kernel(TransposeJob j0, Tr
 // (fp32, may alias dres), optionally hscale*dx as fp16 in fragment order,
 // and this block's dgamma partial sum(dy*x_hat) over its rows.  dy is the sum
 // of S split-K partials (split_stride floats apart), added in order.
-// RB = 2 rows per block, one per 256-thread half, so both rows' loads (dres
-// included) are in flight at once; the halves meet only at the barriers of
-// the reductions and for the dgamma partial (second row's terms via LDS).
-// NIT = D / 2048 rounded up: the feature groups of 8 per thread.
-constexpr int RB = 2;
-template <int S, int NIT>
+// 512 threads, TPR of them per row, so a block's 512 / TPR rows have all their
+// loads (dres included) in flight at once; the rows meet only at the barriers
+// of the reductions and for the dgamma partial (the later rows' terms via LDS,
+// added in row order).  NIT = D / (8 TPR) rounded up: the feature groups of 8
+// per thread.  It is bound by the bytes it moves, so every thread has to carry
+// loads: with 256 threads a row whatever the width, half of them idled at 1024
+// wide, and two rows a block leave twice the dgamma partials of four.
+// Alone (us): 4096 x 1024 20.5 -> 17.2, the sum of its dgamma partials 8.0 -> 5.0;
+// 4096 x 4096 (67) is unchanged.
+template <int S, int TPR, int NIT>
 __global__ __launch_bounds__(512) void rms_backward_kernel(const float* __restrict__ dy, size_t split_stride,
                                                            const float* __restrict__ x,
                                                            const float* __restrict__ gamma, const float* dres,
                                                            float* dx, f16* __restrict__ outh, float hscale,
                                                            float* __restrict__ dg_part, int M, int D, float eps) {
-    __shared__ float red[2][4];
-    __shared__ __attribute__((aligned(16))) float dgs[NIT * 2048];
-    const int half = threadIdx.x >> 8, t = threadIdx.x & 255, w = t >> 6, lane = t & 63;
-    const int row = blockIdx.x * RB + half;
+    constexpr int RB = 512 / TPR, NW = TPR / 64, LD = NIT * 8 * TPR;
+    __shared__ float red[RB][NW];
+    __shared__ __attribute__((aligned(16))) float dgs[RB - 1][LD];
+    const int slot = threadIdx.x / TPR, t = threadIdx.x % TPR, w = t >> 6, lane = t & 63;
+    const int row = blockIdx.x * RB + slot;
     const bool live = row < M;
-    // sum over this half's 4 waves; every thread of the half gets it
-    auto half_sum = [&](float v) {
+    // sum over the row's NW waves; every thread of the row gets it
+    auto row_sum = [&](float v) {
         v = wave_sum(v);
+        if constexpr (NW == 1) return v;
         __syncthreads();
-        if (lane == 0) red[half][w] = v;
+        if (lane == 0) red[slot][w] = v;
         __syncthreads();
-        return (red[half][0] + red[half][1]) + (red[half][2] + red[half][3]);
+        if constexpr (NW == 2) return red[slot][0] + red[slot][1];
+        return (red[slot][0] + red[slot][1]) + (red[slot][NW - 2] + red[slot][NW - 1]);
     };
     const float* xr = x + (size_t)row * D;
     const float* dr = dy + (size_t)row * D;
@@ -158,7 +165,7 @@ __global__ __launch_bounds__(512) void rms_backward_kernel(const float* __restri
     float ss = 0.f;
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        const int i = t * 8 + it * 2048;
+        const int i = t * 8 + it * 8 * TPR;
         dgp[it][0] = dgp[it][1] = f32x4{};
         if (live && i < D) {
             f32x4 p[S][2];
@@ -179,12 +186,12 @@ __global__ __launch_bounds__(512) void rms_backward_kernel(const float* __restri
             }
         }
     }
-    ss = half_sum(ss);
+    ss = row_sum(ss);
     const float r = 1.0f / sqrtf(ss * (1.0f / (float)D) + eps);
     float dot = 0.f;
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        const int i = t * 8 + it * 2048;
+        const int i = t * 8 + it * 8 * TPR;
         if (live && i < D) {
 #pragma unroll
             for (int hh = 0; hh < 2; ++hh)
@@ -196,10 +203,10 @@ __global__ __launch_bounds__(512) void rms_backward_kernel(const float* __restri
                 }
         }
     }
-    dot = half_sum(dot) * (1.0f / (float)D);
+    dot = row_sum(dot) * (1.0f / (float)D);
 #pragma unroll
     for (int it = 0; it < NIT; ++it) {
-        const int i = t * 8 + it * 2048;
+        const int i = t * 8 + it * 8 * TPR;
         if (live && i < D) {
             f16x8 h;
 #pragma unroll
@@ -216,26 +223,30 @@ __global__ __launch_bounds__(512) void rms_backward_kernel(const float* __restri
             if (outh) *(f16x8*)(outh + frag_off(row, i, D)) = h;
         }
     }
-    // dgamma partial of the block: first row's terms + second row's (zero
-    // when the second row is past M)
-    if (half == 1) {
+    // dgamma partial of the block: its rows' terms in order (zero past M)
+    if (slot > 0) {
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
-            const int i = t * 8 + it * 2048;
+            const int i = t * 8 + it * 8 * TPR;
             if (i < D) {
-                *(f32x4*)(dgs + i) = dgp[it][0];
-                *(f32x4*)(dgs + i + 4) = dgp[it][1];
+                *(f32x4*)(dgs[slot - 1] + i) = dgp[it][0];
+                *(f32x4*)(dgs[slot - 1] + i + 4) = dgp[it][1];
             }
         }
     }
     __syncthreads();
-    if (half == 0) {
+    if (slot == 0) {
 #pragma unroll
         for (int it = 0; it < NIT; ++it) {
-            const int i = t * 8 + it * 2048;
+            const int i = t * 8 + it * 8 * TPR;
             if (i < D) {
-                *(f32x4*)(dg_part + (size_t)blockIdx.x * D + i) = dgp[it][0] + *(const f32x4*)(dgs + i);
-                *(f32x4*)(dg_part + (size_t)blockIdx.x * D + i + 4) = dgp[it][1] + *(const f32x4*)(dgs + i + 4);
+#pragma unroll
+                for (int q = 0; q < RB - 1; ++q) {
+                    dgp[it][0] += *(const f32x4*)(dgs[q] + i);
+                    dgp[it][1] += *(const f32x4*)(dgs[q] + i + 4);
+                }
+                *(f32x4*)(dg_part + (size_t)blockIdx.x * D + i) = dgp[it][0];
+                *(f32x4*)(dg_part + (size_t)blockIdx.x * D + i + 4) = dgp[it][1];
             }
         }
     }
@@ -334,26 +345,46 @@ hipError_t launch_transpose_frag2(const f16* src0, f16* dst0, int R0, int C0, co
     return hipGetLastError();
 }
 
-int rms_backward_blocks(int M) { return (M + RB - 1) / RB; }
+// rms_backward_kernel's threads per row: the fewest whose groups of 8 cover a
+// narrow row in one pass.
+static int rms_backward_tpr(int D) { return D <= 512 ? 64 : D <= 1024 ? 128 : 256; }
+
+int rms_backward_blocks(int M, int D) {
+    const int rb = 512 / rms_backward_tpr(D);
+    return (M + rb - 1) / rb;
+}
+
+namespace {
+template <int S>
+hipError_t launch_rms_backward_s(const float* dy, size_t split_stride, const float* x, const float* gamma,
+                                 const float* dres, float* dx, f16* outh, float hscale, float* dg_part, int M, int D,
+                                 float eps, hipStream_t st) {
+    const dim3 grid(rms_backward_blocks(M, D)), block(512);
+#define RH_RB(TPR_, NIT_)                                                                                     \
+    hipLaunchKernelGGL((rms_backward_kernel<S, TPR_, NIT_>), grid, block, 0, st, dy, split_stride, x, gamma,  \
+                       dres, dx, outh, hscale, dg_part, M, D, eps)
+    const int tpr = rms_backward_tpr(D);
+    if (tpr == 64) RH_RB(64, 1);
+    else if (tpr == 128) RH_RB(128, 1);
+    else if (D <= 2048) RH_RB(256, 1);
+    else if (D <= 4096) RH_RB(256, 2);
+    else RH_RB(256, 4);
+#undef RH_RB
+    return hipGetLastError();
+}
+}  // namespace
 
 hipError_t launch_rms_backward(const float* dy, int nsplit, size_t split_stride, const float* x,
                                const float* gamma, const float* dres, float* dx, f16* outh, float hscale,
                                float* dg_part, int M, int D, float eps, hipStream_t st) {
     if (D % 8 != 0 || D > 8192 || nsplit < 1 || nsplit > 8) return hipErrorInvalidValue;
-#define RH_RB(S_)                                                                                             \
-    case S_:                                                                                                  \
-        if (D <= 4096)                                                                                        \
-            hipLaunchKernelGGL((rms_backward_kernel<S_, 2>), dim3(rms_backward_blocks(M)), dim3(512), 0, st,   \
-                               dy, split_stride, x, gamma, dres, dx, outh, hscale, dg_part, M, D, eps);       \
-        else                                                                                                  \
-            hipLaunchKernelGGL((rms_backward_kernel<S_, 4>), dim3(rms_backward_blocks(M)), dim3(512), 0, st,   \
-                               dy, split_stride, x, gamma, dres, dx, outh, hscale, dg_part, M, D, eps);       \
-        break
+#define RH_RB(S_) \
+    case S_: return launch_rms_backward_s<S_>(dy, split_stride, x, gamma, dres, dx, outh, hscale, dg_part, M, D, eps, st)
     switch (nsplit) {
         RH_RB(1); RH_RB(2); RH_RB(3); RH_RB(4); RH_RB(5); RH_RB(6); RH_RB(7); RH_RB(8);
     }
 #undef RH_RB
-    return hipGetLastError();
+    return hipErrorInvalidValue;
 }
 
 hipError_t launch_dgamma_reduce(const float* part, int nblk, int D, float kappa, float* dgamma, bool store,

@@ -151,3 +151,14 @@ def test_attention_backward_lengths(orc, seq):
     w = random_gammas(ModelWeights.normal(cfg, seed=350, std=0.05), 351)
     tok, tgt = tokens_uniform(352 + seq, cfg.vocab, 2, cfg.seq)
     _run(orc, cfg, w, tok, tgt)
+
+
+# RMSNorm backward with 64, 128 and 256 threads a row: widths ending inside a
+# row's groups and on one, and token counts that leave the last block's rows
+# partly empty.
+@pytest.mark.parametrize("heads,hd,seq", [(2, 64, 9), (4, 128, 13), (5, 128, 9), (8, 128, 15), (9, 128, 7)])
+def test_rmsnorm_backward_widths(orc, heads, hd, seq):
+    cfg = small_cfg(dim=heads * hd, hidden=256, heads=heads, hd=hd, nlayers=1, vocab=256, seq=seq)
+    w = random_gammas(ModelWeights.normal(cfg, seed=360, std=0.05), 361)
+    tok, tgt = tokens_uniform(362 + heads, cfg.vocab, 1, cfg.seq)
+    _run(orc, cfg, w, tok, tgt)
