@@ -55,6 +55,50 @@ struct Frag16 {
 };
 
 // ---------------------------------------------------------------------------
+// An operand of a product that contracts over tokens, C[i][j] = sum_t
+// X[t][i] W[t][j], read straight from the token-major fragment order
+// [tokens][features] that the forward and the backward leave it in.  A 1 KB
+// unit holds 16 tokens x 32 features as 16-byte pieces (8 features of a
+// token); 32 tokens x 32 features are two units, u = 2 (feature / 32) + token
+// half, in the place of the two 16-row x 32-k fragments of a row-major
+// operand.  The MFMA wants 8 consecutive tokens of one feature per lane: two
+// transposing LDS reads (ds_read_b64_tr_b16), each of 4 tokens x 16 features
+// per 16 lanes.  The DMA stores the pieces of odd 8-feature columns with their
+// tokens XOR 4, so the 16 lanes' two columns fall into different banks, and so
+// do those of lane groups 0, 1 and 2, 3.
+//
+// This replaces a transposed copy of every operand (one read and one write of
+// each, a launch for every pair); the products' values and order are the same.
+// Forward + backward of a micro-batch with copies -> without, us: two 4096-wide
+// layers, 8 x 512 tokens 10640 -> 10390, 1 x 512 2458 -> 2418; two 2304-wide,
+// 8 x 1024 9340 -> 8965; four 1024-wide, 8 x 1024 5650 -> 5350; four 512-wide,
+// 1 x 128 865 -> 772.
+struct TrOperand {
+    // source offset (halves) within a unit of what DMA lane l stores at 8 l
+    __device__ static int src(int lane) { return (lane ^ (((lane >> 4) & 1) << 2)) * 8; }
+    // lane's address (halves) in a unit pair, units KD * 512 apart, for tokens
+    // 8g + 4hh + 0..3 of features 0..15 (features 16..31: + 256)
+    __device__ static int base(int lane, int hh, int kd) {
+        const int g = lane >> 4, r = lane & 15, b = (r >> 1) & 1;
+        return (g >> 1) * kd * 512 + b * 128 + 64 * (g & 1) + 32 * (hh ^ b) + 8 * (r >> 2) + 4 * (r & 1);
+    }
+    __device__ static f16x8 read(const f16* p0, const f16* p1) {
+        const f16x4 lo = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                       (__attribute__((address_space(3))) s16x4*)p0));
+        const f16x4 hi = __builtin_bit_cast(f16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                                       (__attribute__((address_space(3))) s16x4*)p1));
+        return f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    }
+    // source of unit f of a tile whose first feature is x0 of the product's
+    // count, at token 0, in rows of nf features (units past the last feature
+    // repeat it)
+    __device__ static const f16* unit(const f16* p, int x0, int f, int count, int nf, int lane) {
+        const int fg = min((x0 >> 5) + (f >> 1), ((count + 31) >> 5) - 1);
+        return p + ((size_t)(f & 1) * (nf >> 5) + fg) * 512 + src(lane);
+    }
+};
+
+// ---------------------------------------------------------------------------
 // Tile policy (DTile): operands go global -> LDS by DMA
 // (global_load_lds_dwordx4: 16 bytes per lane land at LDS base + 16 * lane),
 // so no registers stage them and NS = 4 stages of 32 k are in flight (5 for
@@ -76,9 +120,13 @@ struct Frag16 {
 // fragment itself (lane l: row l%16, k 8(l/16)..+7), so each operand is one
 // 1 KB fragment read as is; same tile sizes, operand bytes and accumulator
 // registers, a different output layout (epilogue16).
-template <int WGN, int WGM, int TN, int TM, bool M16 = false, int NS_ = 4>
+//
+// TR: the operands are token-major matrices [K tokens][features] in fragment
+// order (see TrOperand), for the weight gradients, which contract over tokens.
+template <int WGN, int WGM, int TN, int TM, bool M16 = false, int NS_ = 4, bool TR = false>
 struct DTile {
     static_assert(NS_ == 4 || NS_ == 5, "4 or 5 stages");
+    static_assert(!TR || M16, "transposing reads feed 16x16x32 operands");
     static constexpr bool kM16 = M16;
     static constexpr int NA = 2 * TN, NB = 2 * TM;  // 16-wide A / B tiles per wave (M16)
     static constexpr int BN = 32 * TN * WGN, BM = 32 * TM * WGM, NT = 64 * WGN * WGM;
@@ -118,7 +166,11 @@ struct DTile {
         for (int q = 0; q < LPS; ++q) {
             const int f = min(wv * LPS + q, NWF + NXF - 1);
             loff[q] = f * 512;
-            if (f < NWF) {
+            if constexpr (TR) {
+                gp[q] = f < NWF ? TrOperand::unit(a.W, n0, f, a.N, a.trw, lane)
+                                : TrOperand::unit(a.X, m0, f - NWF, a.M, a.trx, lane);
+                gstep[q] = (f < NWF ? a.trw : a.trx) * 32;  // two 16-token unit rows
+            } else if (f < NWF) {
                 const int rb = min((n0 >> 4) + f, ((a.N + 15) >> 4) - 1);
                 gp[q] = a.W + (size_t)rb * K * 16 + lane * 8;
                 gstep[q] = 512;  // one 32-k fragment column of the 16-row block
@@ -131,6 +183,10 @@ struct DTile {
         const int r = lane & 31, h = lane >> 5;
         constexpr int AO = M16 ? NA : TN, BO = M16 ? NB : TM;
         int ao[AO], bo[BO];
+        // TR: this wave's first A and B unit pairs, per token quad (hh); fragment
+        // x is features 16 (x % 2) of the pair x / 2 further on
+        const int ta0 = wn * NA * 512 + TrOperand::base(lane, 0, 1), ta1 = wn * NA * 512 + TrOperand::base(lane, 1, 1);
+        const int tb = (NWF + wm * NB - wn * NA) * 512;
         if constexpr (M16) {
 #pragma unroll
             for (int i = 0; i < NA; ++i) ao[i] = (wn * NA + i) * 512 + 8 * lane;
@@ -158,7 +214,11 @@ struct DTile {
         // operand m of a stage, in the order the interleaved step reads them
         constexpr int NR = M16 ? NA + NB : 2 * (TN + TM);
         auto read1 = [&](const f16* st, Frags& f, int m) {
-            if constexpr (M16) {
+            if constexpr (TR) {
+                const int x = m < NA ? m : m - NA, o = (x & ~1) * 512 + (x & 1) * 256;
+                if (m < NA) f.a[x] = TrOperand::read(st + ta0 + o, st + ta1 + o);
+                else f.b[x] = TrOperand::read(st + (ta0 + tb) + o, st + (ta1 + tb) + o);
+            } else if constexpr (M16) {
                 if (m < NA) f.a[m] = *(const f16x8*)&st[ao[m]];
                 else f.b[m - NA] = *(const f16x8*)&st[bo[m - NA]];
             } else {
@@ -319,7 +379,7 @@ struct DTile {
 // between barriers): 192x128 and 128x128 stay DTiles.  256x128 runs two k
 // slices a stage (32 MFMAs between barriers, as 256x256): 163 -> 157 us at
 // 2048 x 4096 x 11008, 132 -> 129 at 512 x 32000 x 4096.
-template <int WGN, int WGM, int NA_, int NB_, int KD, int NS_>
+template <int WGN, int WGM, int NA_, int NB_, int KD, int NS_, bool TR = false>
 struct PTile {
     static_assert(WGN * WGM == 8 && NA_ % 2 == 0 && (NS_ == 3 || NS_ == 4), "8 waves, 3 or 4 stages");
     static constexpr bool kM16 = true;
@@ -347,19 +407,39 @@ struct PTile {
         const int wn = wv % WGN, wm = wv / WGN, grp = wv >> 2;
         // this wave's DMA units: u = wv * LPS + q over [weight fragments | activation fragments] x KD slices
         const f16* gp[LPS];
+        int gstep[LPS];
 #pragma unroll
         for (int q = 0; q < LPS; ++q) {
             const int u = wv * LPS + q, f = u / KD, d = u % KD;
+            if constexpr (TR) {
+                const int nf = f < NWF ? a.trw : a.trx;
+                gp[q] = (f < NWF ? TrOperand::unit(a.W, n0, f, a.N, nf, lane)
+                                 : TrOperand::unit(a.X, m0, f - NWF, a.M, nf, lane)) +
+                        (size_t)d * nf * 32;
+                gstep[q] = nf * 32 * KD;
+                continue;
+            }
+            gstep[q] = 512 * KD;
             const int rb = f < NWF ? min((n0 >> 4) + f, ((a.N + 15) >> 4) - 1)
                                    : min((m0 >> 4) + f - NWF, ((a.M + 15) >> 4) - 1);
             gp[q] = (f < NWF ? a.W : a.X) + (size_t)rb * a.K * 16 + d * 512 + lane * 8;
         }
         auto dma = [&](int kt, f16* st, int q) {
             __builtin_amdgcn_global_load_lds(
-                (const void*)(gp[q] + (size_t)kt * (512 * KD)),
+                (const void*)(gp[q] + (size_t)kt * (TR ? gstep[q] : 512 * KD)),
                 (__attribute__((address_space(3))) void*)(st + (wv * LPS + q) * 512), 16, 0, 0);
         };
-        const int ao = wn * NA * KD * 512 + 8 * lane, bo = (NWF + wm * NB) * KD * 512 + 8 * lane;
+        const int lo = TR ? 0 : 8 * lane;
+        const int ao = wn * NA * KD * 512 + lo, bo = (NWF + wm * NB) * KD * 512 + lo;
+        const int tr0 = TrOperand::base(lane, 0, KD), tr1 = TrOperand::base(lane, 1, KD);
+        // fragment x (k slice d) of the operand at o
+        auto frag = [&](const f16* st, int o, int x, int d) -> f16x8 {
+            if constexpr (TR) {
+                const f16* p = st + o + ((x & ~1) * KD + d) * 512 + (x & 1) * 256;
+                return TrOperand::read(p + tr0, p + tr1);
+            }
+            return *(const f16x8*)&st[o + (x * KD + d) * 512];
+        };
 #pragma unroll
         for (int i = 0; i < NA; ++i)
 #pragma unroll
@@ -384,9 +464,9 @@ struct PTile {
 #pragma unroll
             for (int d = 0; d < KD; ++d) {
 #pragma unroll
-                for (int j = 0; j < NB; ++j) fb[d][j] = *(const f16x8*)&st[bo + (j * KD + d) * 512];
+                for (int j = 0; j < NB; ++j) fb[d][j] = frag(st, bo, j, d);
 #pragma unroll
-                for (int i = 0; i < NA; ++i) fa[d][i] = *(const f16x8*)&st[ao + (i * KD + d) * 512];
+                for (int i = 0; i < NA; ++i) fa[d][i] = frag(st, ao, i, d);
             }
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -906,15 +986,43 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
 
 size_t gemm_sk_part_floats() { return (size_t)SK_P * 2 * 256 * 256; }
 
-hipError_t launch_gemm_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st) {
-    if (a.K % 128 != 0 || a.N % 4 != 0 || a.M <= 0 || a.N <= 0 || a.ldo < a.N || !a.out_f32)
-        return hipErrorInvalidValue;
-    using Tl = DTile<2, 4, 2, 1, true>;
+namespace {
+template <class Tl>
+hipError_t launch_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st) {
     if (accumulate)
         hipLaunchKernelGGL((gemm_wgrad_kernel<Tl, true>), dim3(SK_P), dim3(Tl::NT + 64 * WG_SW), 0, st, a);
     else
         hipLaunchKernelGGL((gemm_wgrad_kernel<Tl, false>), dim3(SK_P), dim3(Tl::NT + 64 * WG_SW), 0, st, a);
     return hipGetLastError();
+}
+
+template <int EPI>
+hipError_t launch_tokens(const GemmArgs& a, hipStream_t st) {
+    auto go = [&](auto T) {
+        using Tl = decltype(T);
+        const int tiles = ((a.N + Tl::BN - 1) / Tl::BN) * ((a.M + Tl::BM - 1) / Tl::BM);
+        hipLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_DP>), dim3(tiles), dim3(Tl::NT), 0, st, a, 1, 0LL);
+        return hipGetLastError();
+    };
+    switch (a.force_cfg ? a.force_cfg : tile_pick(a.M, a.N, nullptr)) {
+        case GCFG_D8_256x256: return go(PTile<2, 4, 8, 4, 1, 4, true>{});
+        case GCFG_D8_256x128: return go(PTile<4, 2, 4, 4, 2, 3, true>{});
+        case GCFG_D8_192x256: return go(DTile<2, 4, 3, 2, true, 4, true>{});
+        case GCFG_D8_192x128: return go(DTile<2, 4, 3, 1, true, 4, true>{});
+        case GCFG_D8_128x128: return go(DTile<2, 4, 2, 1, true, 4, true>{});
+    }
+    return hipErrorInvalidValue;
+}
+
+bool tr_ok(const GemmArgs& a) { return a.trx >= a.M && a.trw >= a.N && a.trx % 128 == 0 && a.trw % 128 == 0; }
+}  // namespace
+
+hipError_t launch_gemm_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st) {
+    if (a.K % 128 != 0 || a.N % 4 != 0 || a.M <= 0 || a.N <= 0 || a.ldo < a.N || !a.out_f32)
+        return hipErrorInvalidValue;
+    if (a.trx || a.trw)
+        return tr_ok(a) ? launch_wgrad<DTile<2, 4, 2, 1, true, 4, true>>(a, accumulate, st) : hipErrorInvalidValue;
+    return launch_wgrad<DTile<2, 4, 2, 1, true>>(a, accumulate, st);
 }
 
 namespace {
@@ -982,6 +1090,11 @@ hipError_t launch_gemm(int epi, const GemmArgs& a, hipStream_t st) {
                         a.ldo != a.part_cols || a.resid_in || !a.out_part1 ||
                         (a.N > 2 * a.part_cols && !a.out_part2)))
         return hipErrorInvalidValue;
+    if (a.trx || a.trw) {
+        if (!tr_ok(a)) return hipErrorInvalidValue;
+        if (epi == EPI_F32) return launch_tokens<EPI_F32>(a, st);
+        return epi == EPI_RESID ? launch_tokens<EPI_RESID>(a, st) : hipErrorInvalidValue;
+    }
     switch (epi) {
         case EPI_F32: return launch_epi<EPI_F32>(a, st);
         case EPI_RESID: return launch_epi<EPI_RESID>(a, st);

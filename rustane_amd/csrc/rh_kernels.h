@@ -41,6 +41,12 @@ struct GemmArgs {
     // to three outputs [M][ldo = part_cols]: out_f32, out_part1, out_part2.
     int part_cols;
     float *out_part1, *out_part2;
+    // EPI_F32 / EPI_RESID and the weight-gradient kernel: trx, trw > 0 when X
+    // and W are token-major, X [K][trx] and W [K][trw] in fragment order (K
+    // tokens; all three multiples of 128), read as their transposes.  W may
+    // point at feature f (a multiple of 32) of its rows, 16 f halves further,
+    // where N features from f on lie within the row.
+    int trx, trw;
     // Optional timing: stamped at the kernel's own start and end by the
     // one-block-per-tile launch (hipExtLaunchKernelGGL), recorded around the
     // launches otherwise.

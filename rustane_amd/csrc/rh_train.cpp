@@ -17,8 +17,9 @@
 //
 // Every product is an NT GEMM of the forward's kernel: the data-gradient
 // GEMMs stream transposed copies of the weights (built once per weight
-// version), the weight-gradient GEMMs contract over tokens and take
-// token-inner (transposed) copies of their operands, and accumulate into the
+// version), the weight-gradient GEMMs contract over tokens (whole blocks of
+// 128 read in place by transposing LDS reads, ragged counts from token-inner
+// copies of the operands), and accumulate into the
 // fp32 gradients in their epilogue (C += kappa * acc).  Gradients keep the
 // reference's tensor shapes and orientation and accumulate across calls.
 #include "rh_ctx.h"
@@ -58,11 +59,12 @@ struct TrainState {
     // alpha (dffn), H1m = alpha * dx2, H2 = [dh1 | dh3], H2q = [dq | dk | dv].
     f16 *dlh = nullptr, *dlT = nullptr, *H1 = nullptr, *H1m = nullptr, *H2 = nullptr, *H2q = nullptr;
     // The weight-gradient GEMMs run on the side stream in four groups per
-    // layer (0: dW2, 1: dW1 dW3, 2: dWo, 3: dWq dWk dWv), each after its
-    // token-inner operand copies tx[g] (written on the side stream too, from
-    // the activation gradient above and a forward cache).  ready[g] (main):
-    // group g's activation gradient is written; read[g] (side): the copy has
-    // read it, so the main stream may rewrite that buffer a layer later.
+    // layer (0: dW2, 1: dW1 dW3, 2: dWo, 3: dWq dWk dWv), from the activation
+    // gradient above and a forward cache, or for ragged token counts from
+    // token-inner copies of them, tx[g] (written on the side stream too).
+    // ready[g] (main): group g's activation gradient is written; read[g]
+    // (side): it has been read (by the GEMM, or by the copy), so the main
+    // stream may rewrite that buffer a layer later.
     f16* tx[4][2] = {};
     hipStream_t side = nullptr;
     hipEvent_t ready[5] = {}, read[4] = {};  // ready[4]: the logits gradient
@@ -226,7 +228,7 @@ int ensure_train_ws(rh_ctx* ctx, int B, int S) {
     RCK(dalloc(ctx, &T->H1m, m16 * D));
     RCK(dalloc(ctx, &T->H2, m16 * 2 * F));
     RCK(dalloc(ctx, &T->H2q, m16 * 3 * D));
-    const size_t txr[4][2] = {{D, F}, {2 * F, D}, {D, D}, {3 * D, D}};  // rows of each copy
+    const size_t txr[4][2] = {{D, F}, {D, 2 * F}, {D, D}, {D, 3 * D}};  // rows of each copy
     for (int g = 0; g < 4; ++g)
         for (int i = 0; i < 2; ++i) RCK(dalloc(ctx, &T->tx[g][i], txr[g][i] * mp));
     RCK(dalloc(ctx, &T->dOh, m * D));
@@ -329,9 +331,11 @@ int gamma_grad(rh_ctx* ctx, int nblk, int D, float kappa, float* dgamma) {
 // 128x128 31 | 40, 8192 x 1024 256x128 62 | 68.  A short K after a zero leaves
 // the fp32 output most of the time; large outputs then take the kernel whose
 // store waves write a tile while the next one is computed.
+// trx, trw > 0: X and W are token-major instead, [Mp][trx] and [Mp][trw].
 int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* out,
-              hipStream_t st) {
+              hipStream_t st, int trx = 0, int trw = 0) {
     rh::GemmArgs g{};
+    g.trx = trx; g.trw = trw;
     g.X = X; g.W = W; g.M = rows; g.N = cols; g.K = ctx->train->Mp;
     g.out_f32 = out; g.ldo = cols; g.alpha = kappa;
     g.nt_out = true;  // read only by the optimizer
@@ -349,16 +353,18 @@ int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float
 // at K = 4096, dWq..dWv 85 -> 32 us, dW1 dW3 62 -> 50; 4096 wide three products
 // of one round each stay (334 against 358 us).
 int grad_gemms(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* const* out, int n,
-               hipStream_t st) {
-    if (rh::gemm_tile_cost(rows, n * cols) >= (float)n * rh::gemm_tile_cost(rows, cols)) {
+               hipStream_t st, int trx = 0, int trw = 0) {
+    if (n == 1 || rh::gemm_tile_cost(rows, n * cols) >= (float)n * rh::gemm_tile_cost(rows, cols)) {
         for (int j = 0; j < n; ++j)
-            RCK(grad_gemm(ctx, X, W + (size_t)j * cols * ctx->train->Mp, rows, cols, kappa, out[j], st));
+            RCK(grad_gemm(ctx, X, W + (size_t)j * cols * (trw ? 16 : ctx->train->Mp), rows, cols, kappa, out[j], st,
+                          trx, trw));
         return RH_OK;
     }
     rh::GemmArgs g{};
     g.X = X; g.W = W; g.M = rows; g.N = n * cols; g.K = ctx->train->Mp;
     g.out_f32 = out[0]; g.out_part1 = out[1]; g.out_part2 = n > 2 ? out[2] : nullptr;
     g.part_cols = g.ldo = cols; g.alpha = kappa;
+    g.trx = trx; g.trw = trw;
     g.nt_out = true;
     LCK(rh::launch_gemm(ctx->train->zero ? rh::EPI_F32 : rh::EPI_RESID, g, st));
     return RH_OK;
@@ -396,7 +402,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
     const int nblk = rh::rms_backward_blocks(M, D);
     hipStream_t st = ctx->stream;
     // Main stream: the chain through the data gradients.  Side stream: the
-    // weight gradients, each group from its own copies, after the activation
+    // weight gradients, each group after the activation
     // gradient it reads is written (ready) and before that buffer is rewritten
     // a layer later (read).  No buffer either stream writes is touched by the
     // other until the event that orders them.
@@ -414,8 +420,28 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
     // CE gradient (internal units), dx_final = dl E, dembed += dl^T x_final
     LCK(rh::launch_ce_backward(ctx->logits, ctx->d_tgt, T->dlh, M, V, Vp, T->fwd_softcap, rh::GRAD_UNIT, st));
     RCK(publish(4));
-    LCK(rh::launch_transpose_frag2(T->dlh, T->dlT, M, Vp, T->xf, T->tx[0][0], M, D, Mp, sd));
-    RCK(grad_gemm(ctx, T->dlT, T->tx[0][0], V, D, kappa, T->dembed, sd));
+    // Weight gradients contract over tokens.  With whole 128-token blocks the
+    // GEMMs read the token-major activations and their gradients in place
+    // (then read[g] is the GEMM's end), which was 0.3 - 12% faster at every
+    // width (512 - 4096) and token count (128 - 8192) timed; otherwise the rows
+    // past the last token have to be zeros and they take padded token-inner
+    // copies.
+    const bool tr = M == Mp;
+    auto grads = [&](int g, const f16* X, int nx, const f16* W, int nw, int rows, int cols, float* const* out,
+                     int n) -> int {
+        if (!tr) {
+            LCK(rh::launch_transpose_frag2(X, T->tx[g][0], M, nx, W, T->tx[g][1], M, nw, Mp, sd));
+            HCK(hipEventRecord(T->read[g], sd));
+            X = T->tx[g][0];
+            W = T->tx[g][1];
+        }
+        RCK(grad_gemms(ctx, X, W, rows, cols, kappa, out, n, sd, tr ? nx : 0, tr ? nw : 0));
+        if (tr) HCK(hipEventRecord(T->read[g], sd));
+        return RH_OK;
+    };
+    if (!tr) LCK(rh::launch_transpose_frag2(T->dlh, T->dlT, M, Vp, T->xf, T->tx[0][0], M, D, Mp, sd));
+    RCK(grad_gemm(ctx, tr ? T->dlh : T->dlT, tr ? T->xf : T->tx[0][0], V, D, kappa, T->dembed, sd, tr ? Vp : 0,
+                  tr ? D : 0));
     const size_t MD = (size_t)M * D;  // stride of the data-gradient partials
     const float* dp;
     int ns;
@@ -429,15 +455,9 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         const TrainState::Cache& cc = T->c[l];
         const TrainState::WT& wt = T->wt[l];
         float* const* G = T->dlay[l].data();
-        f16* const* X0 = T->tx[0];
-        f16* const* X1 = T->tx[1];
-        f16* const* X2 = T->tx[2];
-        f16* const* X3 = T->tx[3];
         // dW2 += dffn^T gate (side); dgate = dffn W2 with the SiLU backward -> [dh1 | dh3]
         RCK(publish(0));
-        LCK(rh::launch_transpose_frag2(T->H1, X0[0], M, D, cc.gate, X0[1], M, F, Mp, sd));
-        HCK(hipEventRecord(T->read[0], sd));
-        RCK(grad_gemm(ctx, X0[0], X0[1], D, F, kappa, G[6], sd));
+        RCK(grads(0, T->H1, D, cc.gate, F, D, F, G + 6, 1));
         RCK(rewrite(1));
         {
             rh::GemmArgs g{};
@@ -448,9 +468,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         }
         // dx_ffn = [dh1 | dh3] [W1 | W3]^T; dW1, dW3 += x2n^T dh (side)
         RCK(publish(1));
-        LCK(rh::launch_transpose_frag2(T->H2, X1[0], M, 2 * F, cc.x2n, X1[1], M, D, Mp, sd));
-        HCK(hipEventRecord(T->read[1], sd));
-        RCK(grad_gemms(ctx, X1[1], X1[0], D, F, kappa, G + 4, 2, sd));
+        RCK(grads(1, cc.x2n, D, T->H2, 2 * F, D, F, G + 4, 2));
         RCK(data_gemm(ctx, T->H2, wt.w13t, M, D, 2 * F, T->gout, &dp, &ns));
         // dx2 = RMSNorm2'(dx_ffn) + dy (in place in dres); a*dx2 -> H1m
         RCK(rewrite(2));
@@ -459,9 +477,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         RCK(gamma_grad(ctx, nblk, D, kappa, G[8]));
         // da = (a dx2) Wo^T; dWo += attn^T (a dx2) (side)
         RCK(publish(2));
-        LCK(rh::launch_transpose_frag2(T->H1m, X2[0], M, D, cc.attn, X2[1], M, D, Mp, sd));
-        HCK(hipEventRecord(T->read[2], sd));
-        RCK(grad_gemm(ctx, X2[1], X2[0], D, D, kappa, G[3], sd));
+        RCK(grads(2, cc.attn, D, T->H1m, D, D, D, G + 3, 1));
         RCK(data_gemm(ctx, T->H1m, wt.ot, M, D, D, T->gout, &dp, &ns));
         // attention backward -> dq | dk | dv with the RoPE backward, as the fp16
         // operand H2q (rewritten: the side stream has copied the previous layer's)
@@ -470,9 +486,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
                                      ctx->rope, B, H, S, hd, st));
         // dxn = dqkv [Wq | Wk | Wv]^T; dWq, dWk, dWv += xn^T d{q,k,v} (side)
         RCK(publish(3));
-        LCK(rh::launch_transpose_frag2(T->H2q, X3[0], M, 3 * D, cc.xn, X3[1], M, D, Mp, sd));
-        HCK(hipEventRecord(T->read[3], sd));
-        RCK(grad_gemms(ctx, X3[1], X3[0], D, D, kappa, G, 3, sd));
+        RCK(grads(3, cc.xn, D, T->H2q, 3 * D, D, D, G, 3));
         RCK(data_gemm(ctx, T->H2q, wt.qkvt, M, D, 3 * D, T->gout, &dp, &ns));
         // dy' = RMSNorm1'(dxn) + dx2 (in place); a*dy' -> H1 (the next layer's dffn)
         RCK(rewrite(0));

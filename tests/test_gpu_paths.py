@@ -162,3 +162,17 @@ def test_rmsnorm_backward_widths(orc, heads, hd, seq):
     w = random_gammas(ModelWeights.normal(cfg, seed=360, std=0.05), 361)
     tok, tgt = tokens_uniform(362 + heads, cfg.vocab, 1, cfg.seq)
     _run(orc, cfg, w, tok, tgt)
+
+
+# Weight gradients of whole 128-token blocks read the token-major operands in
+# place, others take transposed copies: token counts on both sides, one and
+# several layers (each buffer rewritten a layer after its product read it), and
+# a vocabulary and widths that end inside a tile.
+@pytest.mark.parametrize("heads,hidden,nlayers", [(1, 128, 1), (3, 640, 2), (5, 1408, 3)])
+@pytest.mark.parametrize("batch,seq", [(1, 128), (2, 64), (3, 128), (2, 96)])
+@pytest.mark.parametrize("calls", [1, 2])
+def test_weight_gradients_of_whole_blocks(orc, heads, hidden, nlayers, batch, seq, calls):
+    cfg = small_cfg(dim=128 * heads, hidden=hidden, heads=heads, hd=128, nlayers=nlayers, vocab=520, seq=seq)
+    w = random_gammas(ModelWeights.normal(cfg, seed=370 + heads, std=0.05), 371)
+    tok, tgt = tokens_uniform(372 + seq, cfg.vocab, batch, cfg.seq)
+    _run(orc, cfg, w, tok, tgt, calls=calls)
