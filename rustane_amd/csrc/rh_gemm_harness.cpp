@@ -1,6 +1,6 @@
 // rh_gemm_harness.cpp -- test harness over the prefill GEMM family.
 //
-// Runs one launch_gemm / launch_gemm_resid_norm on host buffers with a forced
+// Runs one launch_gemm / launch_gemm_resid_norm / launch_gemm_wgrad on host buffers with a forced
 // tile configuration, so parity tests can sweep every configuration (data
 // parallel, stream-K, split-K, the 16x16x32 tile) and epilogue on ragged
 // shapes that the shape heuristic would not pick.  Not part of the library's
@@ -8,7 +8,8 @@
 // librustane_gemm_harness.so, which only the tests load.
 //
 // Host operands are fp16 bit patterns already in fragment order (frag_off),
-// W with ceil(N/16)*16 rows and X with ceil(M/16)*16 rows of K halves.
+// W with ceil(N/16)*16 rows and X with ceil(M/16)*16 rows of K halves (the
+// token-major operands of rhh_gemm_grads: K rows of trx and trw halves).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -190,6 +191,54 @@ int rhh_gemm_wgrad(const uint16_t* wf, const uint16_t* xf, int M, int N, int K, 
     if (e != hipSuccess) return (int)e;
     if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
     if (hipMemcpy(io_f32, of, (size_t)M * N * 4, hipMemcpyDeviceToHost) != hipSuccess) return -1;
+    return 0;
+}
+
+// The products of the weight gradients as the backward runs them (no
+// stream-K workspace).  trx, trw > 0: xf is token-major [K][trx] and wf
+// [K][trw], both in fragment order, and the product takes X's features
+// 0..M-1 and W's w_off..w_off+N-1 (w_off a multiple of 32); 0: row-major
+// operands as above.  part_cols > 0: the N features go to up to three outputs
+// [M][part_cols] (io0, io1, io2), else to io0 [M][N].  accumulate: io += alpha
+// * product, else io = alpha * product.  cfg: a GemmCfg value, 0 (the tile
+// model) or -1 (the store-wave kernel: one output, no accumulation).
+int rhh_gemm_grads(int cfg, int accumulate, const uint16_t* wf, const uint16_t* xf, int M, int N, int K, int trx,
+                   int trw, int w_off, float alpha, int part_cols, float* io0, float* io1, float* io2) {
+    if (M <= 0 || N <= 0 || K <= 0 || !wf || !xf || !io0 || w_off < 0 || w_off % 32) return -1;
+    const bool tr = trx > 0;
+    if (tr != (trw > 0) || (tr ? K % 16 || trx < M || trw < w_off + N : w_off != 0)) return -1;
+    if (part_cols ? part_cols < 0 || N > 3 * part_cols || (N > part_cols && !io1) || (N > 2 * part_cols && !io2)
+                  : io1 || io2)
+        return -1;
+    if (cfg < 0 && (part_cols || accumulate)) return -1;
+    Dev d;
+    const size_t wn = tr ? (size_t)K * trw : (size_t)up16(N) * K, xn = tr ? (size_t)K * trx : (size_t)up16(M) * K;
+    const int cols = part_cols ? part_cols : N;
+    f16* W = d.alloc<f16>(wn);
+    f16* X = d.alloc<f16>(xn);
+    if (!W || !X || hipMemcpy(W, wf, wn * 2, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(X, xf, xn * 2, hipMemcpyHostToDevice) != hipSuccess)
+        return -1;
+    float* const io[3] = {io0, io1, io2};
+    float* out[3] = {};
+    const size_t on = (size_t)M * cols;
+    for (int i = 0; i < 3; ++i) {
+        if (!io[i]) continue;
+        out[i] = d.alloc<float>(on);
+        if (!out[i] || hipMemcpy(out[i], io[i], on * 4, hipMemcpyHostToDevice) != hipSuccess) return -1;
+    }
+    rh::GemmArgs a{};
+    a.W = W + (size_t)w_off * 16; a.X = X; a.M = M; a.N = N; a.K = K;
+    a.trx = trx; a.trw = trw;
+    a.out_f32 = out[0]; a.out_part1 = out[1]; a.out_part2 = out[2];
+    a.part_cols = part_cols; a.ldo = cols; a.alpha = alpha; a.nt_out = true;
+    a.force_cfg = cfg > 0 ? cfg : 0;
+    hipError_t e = cfg < 0 ? rh::launch_gemm_wgrad(a, false, nullptr)
+                           : rh::launch_gemm(accumulate ? rh::EPI_RESID : rh::EPI_F32, a, nullptr);
+    if (e != hipSuccess) return (int)e;
+    if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
+    for (int i = 0; i < 3; ++i)
+        if (out[i] && hipMemcpy(io[i], out[i], on * 4, hipMemcpyDeviceToHost) != hipSuccess) return -1;
     return 0;
 }
 

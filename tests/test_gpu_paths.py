@@ -2,6 +2,8 @@
 where a variant's tiles, remainders or limits can go wrong, and is checked
 against the CPU oracle or a float64 product, at the bars of the tests of the
 same path."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -132,14 +134,81 @@ def test_decode_attention_chunks(hd, max_ctx, p0):
 
 
 # Weight gradients of one input as one product with two or three outputs
-# (narrow models): tiles that straddle the outputs, stored and accumulated.
-@pytest.mark.parametrize("heads,hidden", [(1, 128), (3, 640), (5, 1408)])
+# (narrow models), stored and accumulated: 128-wide tiles, whose edges fall on
+# the outputs' edges, and dW1 | dW3 of 1024 x 2816 on 192-wide tiles, which
+# straddle the two outputs.
+@pytest.mark.parametrize("heads,hidden", [(1, 128), (3, 640), (5, 1408), (8, 2816)])
 @pytest.mark.parametrize("calls", [1, 2])
 def test_joint_weight_gradients(orc, heads, hidden, calls):
     cfg = small_cfg(dim=128 * heads, hidden=hidden, heads=heads, hd=128, nlayers=1, vocab=512, seq=70)
     w = random_gammas(ModelWeights.normal(cfg, seed=340 + heads, std=0.05), 341)
     tok, tgt = tokens_uniform(342, cfg.vocab, 2, cfg.seq)
     _run(orc, cfg, w, tok, tgt, calls=calls)
+
+
+def grads_product(lib, cfg, accumulate, x, w, M, N, alpha, outs, part_cols=0, w_off=0, tokens=False):  # noqa: F811
+    """x, w: [K][features] with tokens, else [M][K] and [N][K]; outs: one to three output arrays."""
+    f, i, p = ctypes.c_float, ctypes.c_int, ctypes.c_void_p
+    lib.rhh_gemm_grads.argtypes = [i, i, p, p, i, i, i, i, i, i, f, i, p, p, p]
+    K = x.shape[0] if tokens else x.shape[1]
+    io = list(outs) + [None] * (3 - len(outs))
+    xf, wf = frag_pack(x), frag_pack(w)
+    rc = lib.rhh_gemm_grads(cfg, accumulate, ptr(wf), ptr(xf), M, N, K, x.shape[1] if tokens else 0,
+                            w.shape[1] if tokens else 0, w_off, alpha, part_cols, *[ptr(o) for o in io])
+    assert rc == 0, f"rhh_gemm_grads cfg {cfg}: error {rc}"
+
+
+PICKED = ["D8_256x256", "D8_256x128", "D8_192x256", "D8_192x128", "D8_128x128"]  # the tile model's choices
+
+
+# Products over tokens with both operands token-major, every tile the model can
+# pick and the store-wave kernel: outputs that end inside a tile and inside a
+# 32-feature block, operand rows wider than the product and a W that starts
+# inside its rows (dW3's), k loops shorter than the stage rings and ending on
+# each of their buffers, and more tiles than blocks or groups of 8 M-tiles.
+# fp32 sums of K <= 640 products: 1e-5 of max|Y|.
+@pytest.mark.parametrize("M,N,K,trx,trw,w_off", [(4, 4, 128, 128, 128, 0), (600, 700, 128, 640, 768, 32),
+                                                 (300, 1000, 256, 384, 1152, 96), (600, 700, 384, 640, 768, 64),
+                                                 (300, 516, 640, 384, 640, 0), (2100, 2200, 128, 2176, 2304, 0)])
+@pytest.mark.parametrize("name", PICKED + ["store_waves"])
+def test_products_over_tokens(lib, name, M, N, K, trx, trw, w_off):  # noqa: F811
+    rng = np.random.default_rng(28)
+    x, w = (rng.standard_normal((K, n)).astype(np.float16) for n in (trx, trw))
+    y = x[:, :M].T.astype(np.float64) @ w[:, w_off:w_off + N].astype(np.float64)
+    cfg = CFGS.get(name, -1)
+    out = np.full((M, N), np.nan, np.float32)
+    grads_product(lib, cfg, 0, x, w, M, N, 0.5, [out], w_off=w_off, tokens=True)
+    close(out, 0.5 * y, 1e-5, f"{name} store")
+    if cfg < 0:
+        return
+    x0 = rng.standard_normal((M, N)).astype(np.float32)
+    io = x0.copy()
+    grads_product(lib, cfg, 1, x, w, M, N, 0.25, [io], w_off=w_off, tokens=True)
+    close(io, x0.astype(np.float64) + 0.25 * y, 1e-5, f"{name} accumulate")
+
+
+# One product with two or three outputs: output widths below, at and past a
+# tile's, so that tiles hold features of two or three outputs, and a last one
+# cut short, whose remaining columns stay as they are.
+@pytest.mark.parametrize("tokens", [False, True])
+@pytest.mark.parametrize("part_cols,N", [(128, 384), (132, 264), (132, 396), (320, 640), (320, 900), (68, 204)])
+@pytest.mark.parametrize("name", PICKED)
+def test_products_with_several_outputs(lib, name, part_cols, N, tokens):  # noqa: F811
+    M, K = 300, 256
+    rng = np.random.default_rng(29)
+    x = rng.standard_normal((K, 384) if tokens else (M, K)).astype(np.float16)
+    w = rng.standard_normal((K, (N + 127) // 128 * 128) if tokens else (N, K)).astype(np.float16)
+    xd, wd = (x[:, :M].T, w[:, :N].T) if tokens else (x, w)
+    y = xd.astype(np.float64) @ wd.astype(np.float64).T
+    n = (N + part_cols - 1) // part_cols
+    old = rng.standard_normal((n, M, part_cols)).astype(np.float32)
+    for accumulate in (0, 1):
+        outs = [o.copy() for o in old]
+        grads_product(lib, CFGS[name], accumulate, x, w, M, N, 0.5, outs, part_cols=part_cols, tokens=tokens)
+        got = np.concatenate(outs, 1)
+        before = np.concatenate(list(old), 1)
+        assert np.array_equal(got[:, N:], before[:, N:])
+        close(got[:, :N], before[:, :N].astype(np.float64) * accumulate + 0.5 * y, 1e-5, f"{name} accumulate {accumulate}")
 
 
 # Attention backward at head dim 128: lengths that end inside and on a 64-row
@@ -166,9 +235,10 @@ def test_rmsnorm_backward_widths(orc, heads, hd, seq):
 
 # Weight gradients of whole 128-token blocks read the token-major operands in
 # place, others take transposed copies: token counts on both sides, one and
-# several layers (each buffer rewritten a layer after its product read it), and
-# a vocabulary and widths that end inside a tile.
-@pytest.mark.parametrize("heads,hidden,nlayers", [(1, 128, 1), (3, 640, 2), (5, 1408, 3)])
+# several layers (each buffer rewritten a layer after its product read it), a
+# vocabulary that ends inside a tile, and (8, 2816), whose dW1 | dW3 runs on
+# 192-wide tiles that straddle the outputs.
+@pytest.mark.parametrize("heads,hidden,nlayers", [(1, 128, 1), (3, 640, 2), (5, 1408, 3), (8, 2816, 1)])
 @pytest.mark.parametrize("batch,seq", [(1, 128), (2, 64), (3, 128), (2, 96)])
 @pytest.mark.parametrize("calls", [1, 2])
 def test_weight_gradients_of_whole_blocks(orc, heads, hidden, nlayers, batch, seq, calls):
