@@ -987,12 +987,9 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
 size_t gemm_sk_part_floats() { return (size_t)SK_P * 2 * 256 * 256; }
 
 namespace {
-template <class Tl>
-hipError_t launch_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st) {
-    if (accumulate)
-        hipLaunchKernelGGL((gemm_wgrad_kernel<Tl, true>), dim3(SK_P), dim3(Tl::NT + 64 * WG_SW), 0, st, a);
-    else
-        hipLaunchKernelGGL((gemm_wgrad_kernel<Tl, false>), dim3(SK_P), dim3(Tl::NT + 64 * WG_SW), 0, st, a);
+template <class Tl, bool ACC>
+hipError_t launch_wgrad(const GemmArgs& a, hipStream_t st) {
+    hipLaunchKernelGGL((gemm_wgrad_kernel<Tl, ACC>), dim3(SK_P), dim3(Tl::NT + 64 * WG_SW), 0, st, a);
     return hipGetLastError();
 }
 
@@ -1020,9 +1017,11 @@ bool tr_ok(const GemmArgs& a) { return a.trx >= a.M && a.trw >= a.N && a.trx % 1
 hipError_t launch_gemm_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st) {
     if (a.K % 128 != 0 || a.N % 4 != 0 || a.M <= 0 || a.N <= 0 || a.ldo < a.N || !a.out_f32)
         return hipErrorInvalidValue;
+    using Tl = DTile<2, 4, 2, 1, true>;
     if (a.trx || a.trw)
-        return tr_ok(a) ? launch_wgrad<DTile<2, 4, 2, 1, true, 4, true>>(a, accumulate, st) : hipErrorInvalidValue;
-    return launch_wgrad<DTile<2, 4, 2, 1, true>>(a, accumulate, st);
+        return tr_ok(a) && !accumulate ? launch_wgrad<DTile<2, 4, 2, 1, true, 4, true>, false>(a, st)
+                                       : hipErrorInvalidValue;
+    return accumulate ? launch_wgrad<Tl, true>(a, st) : launch_wgrad<Tl, false>(a, st);
 }
 
 namespace {

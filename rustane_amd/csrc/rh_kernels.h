@@ -111,7 +111,8 @@ hipError_t launch_gemm_partials(const GemmArgs& a, int* nsplit, hipStream_t st);
 // Weight-gradient GEMM for a short K (the token count): out [M][ldo] fp32 =
 // alpha * X W^T (alpha 0: unscaled), or += when accumulate; persistent blocks
 // whose store waves write each 128x128 tile while the next one is computed.
-// Needs K % 128 == 0, N % 4 == 0.
+// Needs K % 128 == 0, N % 4 == 0.  The backward only stores; token-major
+// operands (trx, trw) are not built to accumulate.
 hipError_t launch_gemm_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st);
 
 // ---------------- attention ----------------
