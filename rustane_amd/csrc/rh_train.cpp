@@ -321,6 +321,11 @@ int gamma_grad(rh_ctx* ctx, int nblk, int D, float kappa, float* dgamma) {
     return RH_OK;
 }
 
+// Whether the store-wave kernel takes the first store of a gradient [rows][cols].
+bool store_waves(const rh_ctx* ctx, int rows, int cols) {
+    return ctx->train->zero && ctx->train->Mp <= 1024 && (size_t)rows * cols >= (size_t)4096 * 4096;
+}
+
 // C[rows][cols] += kappa * X W^T with X [rows][Mp], W [cols][Mp] (token-inner).
 // When every gradient is still zero the epilogue stores kappa * acc instead
 // (the same values; it skips reading the fp32 gradient back).  The tile model
@@ -339,7 +344,7 @@ int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float
     g.X = X; g.W = W; g.M = rows; g.N = cols; g.K = ctx->train->Mp;
     g.out_f32 = out; g.ldo = cols; g.alpha = kappa;
     g.nt_out = true;  // read only by the optimizer
-    if (ctx->train->zero && g.K <= 1024 && (size_t)rows * cols >= (size_t)4096 * 4096) {
+    if (store_waves(ctx, rows, cols)) {
         LCK(rh::launch_gemm_wgrad(g, false, st));
         return RH_OK;
     }
@@ -351,10 +356,17 @@ int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float
 // dWq | dWk | dWv and dW1 | dW3.  As one product with n outputs where that
 // fills the CUs better than n products (the tile model's estimate): 1024 wide
 // at K = 4096, dWq..dWv 85 -> 32 us, dW1 dW3 62 -> 50; 4096 wide three products
-// of one round each stay (334 against 358 us).
+// of one round each stay (334 against 358 us).  Outputs whose first store the
+// store-wave kernel takes stay n products up to 512 tokens, where writing them
+// is most of the time: forward + backward of two layers after a zero, 128 / 256
+// / 512 tokens, joint -> n products, us: 2560 wide 864 -> 854, 979 -> 961, 1228
+// -> 1210, 3072 wide 1009 -> 995, 1127 -> 1112, 1522 -> 1494, 5120 wide 1775 ->
+// 1702, 2162 -> 2096, 3036 -> 3069 (1024 tokens: 1846 -> 1857, 2242 -> 2212 and
+// 4954 -> 5180).
 int grad_gemms(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* const* out, int n,
                hipStream_t st, int trx = 0, int trw = 0) {
-    if (n == 1 || rh::gemm_tile_cost(rows, n * cols) >= (float)n * rh::gemm_tile_cost(rows, cols)) {
+    if (n == 1 || (ctx->train->Mp <= 512 && store_waves(ctx, rows, cols)) ||
+        rh::gemm_tile_cost(rows, n * cols) >= (float)n * rh::gemm_tile_cost(rows, cols)) {
         for (int j = 0; j < n; ++j)
             RCK(grad_gemm(ctx, X, W + (size_t)j * cols * (trw ? 16 : ctx->train->Mp), rows, cols, kappa, out[j], st,
                           trx, trw));

@@ -146,6 +146,25 @@ def test_joint_weight_gradients(orc, heads, hidden, calls):
     _run(orc, cfg, w, tok, tgt, calls=calls)
 
 
+# 2560 x 6912: up to 512 tokens the first dW1 and dW3 are two products of the
+# store-wave kernel, later ones (and longer first ones) one product with two
+# outputs.  Both sum the tokens in order, and with powers of two for the loss
+# scale and the length every scaling is exact: a second call on the same batch
+# doubles the gradients to the bit.
+@pytest.mark.parametrize("seq", [128, 256, 512, 1024])
+def test_first_and_joint_weight_gradients_agree(seq):
+    cfg = small_cfg(dim=2560, hidden=6912, heads=20, hd=128, nlayers=1, vocab=512, seq=seq)
+    tok, tgt = tokens_uniform(343, cfg.vocab, 1, seq)
+    with hb.Context(cfg.to_rh(), 0, 1, 0) as c:
+        c.init_normal(344, 0.02)
+        c.forward_backward(tok, tgt, 256.0)
+        first = c.read_grads()[2][0]
+        c.forward_backward(tok, tgt, 256.0)
+        second = c.read_grads()[2][0]
+    for j in range(7):
+        assert first[j].any() and np.array_equal(second[j], 2 * first[j]), j
+
+
 def grads_product(lib, cfg, accumulate, x, w, M, N, alpha, outs, part_cols=0, w_off=0, tokens=False):  # noqa: F811
     """x, w: [K][features] with tokens, else [M][K] and [N][K]; outs: one to three output arrays."""
     f, i, p = ctypes.c_float, ctypes.c_int, ctypes.c_void_p
