@@ -143,6 +143,13 @@ int dalloc(rh_ctx* ctx, T** p, size_t elems) {
     return RH_OK;
 }
 void dfree(rh_ctx* ctx, void* p);
+// Frees p's buffer and forgets it, so that no later call reads or frees it
+// again when what was to take its place cannot be allocated.
+template <typename T>
+void drop(rh_ctx* ctx, T*& p) {
+    dfree(ctx, p);
+    p = nullptr;
+}
 
 // Launches fn(); when profiling class cls is on (and no graph is being
 // captured) times it with an event pair.  A launcher that takes the two

@@ -53,12 +53,17 @@ int ensure_rope(rh_ctx* ctx, int npos) {
             const float th = (float)p / std::pow(ctx->cfg.rope_base, 2.0f * (float)i / (float)hd);
             t[(size_t)p * (hd / 2) + i] = make_float2(std::cos(th), std::sin(th));
         }
+    float2* fresh = nullptr;  // the old table stays until this one is there: decode steps read it unasked
+    RCK(dalloc(ctx, &fresh, t.size()));
+    const hipError_t e = hipMemcpy(fresh, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice);
+    if (e != hipSuccess) {
+        dfree(ctx, fresh);
+        return fail(ctx, RH_EDEVICE, std::string("copy of the RoPE table: ") + hipGetErrorString(e));
+    }
     HCK(hipStreamSynchronize(ctx->stream));
     drop_graphs(ctx);  // captured steps hold the old table's address
     dfree(ctx, ctx->rope);
-    ctx->rope = nullptr;
-    RCK(dalloc(ctx, &ctx->rope, t.size()));
-    HCK(hipMemcpy(ctx->rope, t.data(), t.size() * sizeof(float2), hipMemcpyHostToDevice));
+    ctx->rope = fresh;
     ctx->rope_len = npos;
     return RH_OK;
 }
@@ -80,9 +85,10 @@ int ensure_workspace(rh_ctx* ctx, int M) {
     if (M <= ctx->ws_M) return RH_OK;
     HCK(hipStreamSynchronize(ctx->stream));
     drop_graphs(ctx);  // captured forwards hold the old buffers' addresses
-    void* olds[] = {ctx->x, ctx->xn, ctx->q, ctx->kbuf, ctx->vbuf, ctx->attn, ctx->gate,
-                    ctx->logits, ctx->tok_loss, ctx->mean, ctx->d_tok, ctx->d_tgt};
-    for (void* p : olds) dfree(ctx, p);
+    ctx->ws_M = 0;  // until every buffer below is there
+    drop(ctx, ctx->x); drop(ctx, ctx->xn); drop(ctx, ctx->q); drop(ctx, ctx->kbuf); drop(ctx, ctx->vbuf);
+    drop(ctx, ctx->attn); drop(ctx, ctx->gate); drop(ctx, ctx->logits); drop(ctx, ctx->tok_loss);
+    drop(ctx, ctx->mean); drop(ctx, ctx->d_tok); drop(ctx, ctx->d_tgt);
     const size_t D = D_(ctx), F = F_(ctx), V = V_(ctx), m = (size_t)M;
     // GEMM operands (xn, attn, gate) are in fragment order: rows padded to 16
     const size_t m16 = (m + 15) / 16 * 16;
@@ -109,8 +115,8 @@ int ensure_workspace(rh_ctx* ctx, int M) {
 int ensure_staging(rh_ctx* ctx, size_t elems) {
     if (elems <= ctx->staging_elems) return RH_OK;
     HCK(hipStreamSynchronize(ctx->stream));
-    dfree(ctx, ctx->staging);
-    ctx->staging = nullptr;
+    drop(ctx, ctx->staging);
+    ctx->staging_elems = 0;
     RCK(dalloc(ctx, &ctx->staging, elems));
     ctx->staging_elems = elems;
     return RH_OK;
