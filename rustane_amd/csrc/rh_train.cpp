@@ -38,12 +38,13 @@ struct TrainState {
     int M = 0, Mp = 0, B = 0, S = 0;
     uint64_t packs_gen = 0;            // weight version the transposed copies hold
     bool zero = true;  // every gradient is 0: the weight-gradient GEMMs store instead of accumulating
+    bool have_static = false;  // the gradients and transposed weights below are allocated
     // fp32 gradients, reference orientation (RSTK order per layer)
     float *dembed = nullptr, *dgf = nullptr;
-    std::vector<std::array<float*, 9>> dlay;
+    std::vector<std::array<float*, 9>> dlay;  // value-initialised: null until allocated
     // transposed fp16 weights (fragment order)
     f16* embed_t = nullptr;  // [D][Vp]
-    struct WT { f16 *qkvt, *ot, *w13t, *w2t; };
+    struct WT { f16 *qkvt = nullptr, *ot = nullptr, *w13t = nullptr, *w2t = nullptr; };
     std::vector<WT> wt;
     // per-layer forward caches
     struct Cache {
@@ -140,39 +141,43 @@ int ensure_train_host(rh_ctx* ctx) {
     return ctx->train ? RH_OK : fail(ctx, RH_ENOMEM, "out of host memory");
 }
 
-// Gradients and transposed weights: allocated once per context.
+// Gradients and transposed weights: allocated once per context (a call that
+// could not allocate them all is continued by the next).
 int ensure_train_static(rh_ctx* ctx) {
     RCK(ensure_train_host(ctx));
     TrainState* T = ctx->train;
-    if (T->dembed) return RH_OK;
+    if (T->have_static) return RH_OK;
     const rh_config& c = ctx->cfg;
     const size_t D = c.dim, F = c.hidden, V = c.vocab, Vp = round_up(V, 128);
-    if (!T->side) {  // the weight-gradient GEMMs' stream (default priority, like the context's)
+    if (!T->side)  // the weight-gradient GEMMs' stream (default priority, like the context's)
         HCK(hipStreamCreateWithFlags(&T->side, hipStreamNonBlocking));
-        for (hipEvent_t& e : T->ready) HCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-        for (hipEvent_t& e : T->read) HCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
-    }
-    RCK(dalloc(ctx, &T->dembed, V * D));
-    RCK(dalloc(ctx, &T->dgf, D));
+    for (hipEvent_t& e : T->ready)
+        if (!e) HCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    for (hipEvent_t& e : T->read)
+        if (!e) HCK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    auto once = [&](auto*& p, size_t n) { return p ? RH_OK : dalloc(ctx, &p, n); };
+    RCK(once(T->dembed, V * D));
+    RCK(once(T->dgf, D));
     T->dlay.resize(c.nlayers);
     const size_t sz[9] = {D * D, D * D, D * D, D * D, D * F, D * F, D * F, D, D};
     size_t nparts = rh::sumsq_blocks(V * D) + rh::sumsq_blocks(D);
     for (auto& g : T->dlay)
         for (int j = 0; j < 9; ++j) {
-            RCK(dalloc(ctx, &g[j], sz[j]));
+            RCK(once(g[j], sz[j]));
             nparts += rh::sumsq_blocks(sz[j]);
         }
-    RCK(dalloc(ctx, &T->norm_part, nparts));
-    RCK(dalloc(ctx, &T->norm_sum, 1));
-    RCK(dalloc(ctx, &T->embed_t, D * Vp));
+    RCK(once(T->norm_part, nparts));
+    RCK(once(T->norm_sum, 1));
+    RCK(once(T->embed_t, D * Vp));
     T->wt.resize(c.nlayers);
     for (auto& w : T->wt) {
-        RCK(dalloc(ctx, &w.qkvt, D * 3 * D));
-        RCK(dalloc(ctx, &w.ot, D * D));
-        RCK(dalloc(ctx, &w.w13t, D * 2 * F));
-        RCK(dalloc(ctx, &w.w2t, F * D));
+        RCK(once(w.qkvt, D * 3 * D));
+        RCK(once(w.ot, D * D));
+        RCK(once(w.w13t, D * 2 * F));
+        RCK(once(w.w2t, F * D));
     }
     T->zero = true;
+    T->have_static = true;
     return RH_OK;
 }
 
@@ -188,21 +193,17 @@ int ensure_train_ws(rh_ctx* ctx, int B, int S) {
     }
     HCK(hipStreamSynchronize(ctx->stream));
     if (T->side) HCK(hipStreamSynchronize(T->side));  // the weight-gradient stream reads some of them
-    // free the old per-shape buffers
+    // free the old per-shape buffers; no capacity until every new one is there
+    T->M = 0;
     for (auto& cc : T->c) {
-        void* ps[] = {cc.xin, cc.x2, cc.lse, cc.xn, cc.q, cc.k, cc.v, cc.attn, cc.x2n, cc.h13, cc.gate};
-        for (void* p : ps) dfree(ctx, p);
+        drop(ctx, cc.xin); drop(ctx, cc.x2); drop(ctx, cc.lse); drop(ctx, cc.xn); drop(ctx, cc.q); drop(ctx, cc.k);
+        drop(ctx, cc.v); drop(ctx, cc.attn); drop(ctx, cc.x2n); drop(ctx, cc.h13); drop(ctx, cc.gate);
     }
-    {
-        void* ps[] = {T->xlast, T->xf, T->dlh, T->dlT, T->H1, T->H1m, T->H2, T->H2q, T->dOh,
-                      T->gout, T->dres, T->Drow, T->dgp, T->utok, T->ustart, T->uidx};
-        for (void* p : ps) dfree(ctx, p);
-        for (auto& pr : T->tx)
-            for (f16*& p : pr) {
-                dfree(ctx, p);
-                p = nullptr;
-            }
-    }
+    drop(ctx, T->xlast); drop(ctx, T->xf); drop(ctx, T->dlh); drop(ctx, T->dlT); drop(ctx, T->H1); drop(ctx, T->H1m);
+    drop(ctx, T->H2); drop(ctx, T->H2q); drop(ctx, T->dOh); drop(ctx, T->gout); drop(ctx, T->dres);
+    drop(ctx, T->Drow); drop(ctx, T->dgp); drop(ctx, T->utok); drop(ctx, T->ustart); drop(ctx, T->uidx);
+    for (auto& pr : T->tx)
+        for (f16*& p : pr) drop(ctx, p);
     const rh_config& c = ctx->cfg;
     const size_t D = c.dim, F = c.hidden, V = c.vocab, Vp = round_up(V, 128);
     const size_t m = M, m16 = round_up(m, 16), mp = round_up(m, 128);
@@ -614,16 +615,17 @@ int ensure_opt(rh_ctx* ctx) {
     tensor_sizes(c, sz);
     hipStream_t st = ctx->stream;
     if (!o->moments) {
-        RCK(dalloc(ctx, &o->emb_m, V * D));
-        RCK(dalloc(ctx, &o->emb_v, V * D));
-        RCK(dalloc(ctx, &o->gf_m, D));
-        RCK(dalloc(ctx, &o->gf_v, D));
+        auto once = [&](float*& p, size_t n) { return p ? RH_OK : dalloc(ctx, &p, n); };
+        RCK(once(o->emb_m, V * D));
+        RCK(once(o->emb_v, V * D));
+        RCK(once(o->gf_m, D));
+        RCK(once(o->gf_v, D));
         o->m.resize(c.nlayers);
         o->v.resize(c.nlayers);
         for (int l = 0; l < c.nlayers; ++l)
             for (int j = 0; j < 9; ++j) {
-                RCK(dalloc(ctx, &o->m[l][j], sz[j]));
-                RCK(dalloc(ctx, &o->v[l][j], sz[j]));
+                RCK(once(o->m[l][j], sz[j]));
+                RCK(once(o->v[l][j], sz[j]));
             }
         o->moments = true;
         RCK(zero_moments(ctx));
@@ -674,7 +676,7 @@ float rh_learning_rate(uint32_t step, const rh_train_config* tc) {
 int rh_grad_norm(rh_ctx* ctx, float* norm_out) {
     if (!ctx || !norm_out) return fail(ctx, RH_EINVAL, "null argument");
     TrainState* T = ctx->train;
-    if (!T || !T->dembed || T->zero) {
+    if (!T || !T->have_static || T->zero) {
         *norm_out = 0.f;
         return RH_OK;
     }
@@ -993,7 +995,7 @@ void rh_forward_result_free(rh_forward_result* fwd) { delete fwd; }
 int rh_read_grads_f32(rh_ctx* ctx, float* dembed, float* dgamma_final, float* const* layer_grads) {
     if (!ctx) return RH_EINVAL;
     TrainState* T = ctx->train;
-    if (!T || !T->dembed) return fail(ctx, RH_ESTATE, "no gradients: run rh_forward_backward first");
+    if (!T || !T->have_static) return fail(ctx, RH_ESTATE, "no gradients: run rh_forward_backward first");
     HCK(hipSetDevice(ctx->device));
     const rh_config& c = ctx->cfg;
     const size_t D = c.dim, F = c.hidden, V = c.vocab;
