@@ -58,15 +58,16 @@ struct TrainState {
     // Activation gradients in fp16 fragment order, one buffer per role so each
     // is rewritten only once per layer: H1 = the layer's output gradient times
     // alpha (dffn), H1m = alpha * dx2, H2 = [dh1 | dh3], H2q = [dq | dk | dv].
-    f16 *dlh = nullptr, *dlT = nullptr, *H1 = nullptr, *H1m = nullptr, *H2 = nullptr, *H2q = nullptr;
+    f16 *dlh = nullptr, *H1 = nullptr, *H1m = nullptr, *H2 = nullptr, *H2q = nullptr;
     // The weight-gradient GEMMs run on the side stream in four groups per
     // layer (0: dW2, 1: dW1 dW3, 2: dWo, 3: dWq dWk dWv), from the activation
     // gradient above and a forward cache, or for ragged token counts from
-    // token-inner copies of them, tx[g] (written on the side stream too).
+    // token-inner copies of them, tx[g] and dlT (written on the side stream too).
     // ready[g] (main): group g's activation gradient is written; read[g]
     // (side): it has been read (by the GEMM, or by the copy), so the main
     // stream may rewrite that buffer a layer later.
-    f16* tx[4][2] = {};
+    f16 *tx[4][2] = {}, *dlT = nullptr;
+    int txM = 0;  // token capacity of the copies (0: none allocated)
     hipStream_t side = nullptr;
     hipEvent_t ready[5] = {}, read[4] = {};  // ready[4]: the logits gradient
     f16* dOh = nullptr;
@@ -181,6 +182,32 @@ int ensure_train_static(rh_ctx* ctx) {
     return RH_OK;
 }
 
+void drop_copies(rh_ctx* ctx) {
+    TrainState* T = ctx->train;
+    T->txM = 0;
+    drop(ctx, T->dlT);
+    for (auto& pr : T->tx)
+        for (f16*& p : pr) drop(ctx, p);
+}
+
+// The token-inner copies, which only token counts that are no multiple of 128
+// need (0.8 GB at 4096 wide, vocabulary 32000 and 4096 tokens): sized for the
+// buffers' capacity by the first such call.
+int ensure_copies(rh_ctx* ctx) {
+    TrainState* T = ctx->train;
+    if (T->B * T->S == T->Mp || T->txM >= T->M) return RH_OK;
+    HCK(hipStreamSynchronize(T->side));  // reads them
+    drop_copies(ctx);
+    const rh_config& c = ctx->cfg;
+    const size_t D = c.dim, F = c.hidden, Vp = round_up(c.vocab, 128), mp = round_up(T->M, 128);
+    RCK(dalloc(ctx, &T->dlT, Vp * mp));
+    const size_t rows[4][2] = {{D, F}, {D, 2 * F}, {D, D}, {D, 3 * D}};
+    for (int g = 0; g < 4; ++g)
+        for (int i = 0; i < 2; ++i) RCK(dalloc(ctx, &T->tx[g][i], rows[g][i] * mp));
+    T->txM = T->M;
+    return RH_OK;
+}
+
 // Caches and workspace for B sequences of S tokens (grow-only).
 int ensure_train_ws(rh_ctx* ctx, int B, int S) {
     TrainState* T = ctx->train;
@@ -199,11 +226,10 @@ int ensure_train_ws(rh_ctx* ctx, int B, int S) {
         drop(ctx, cc.xin); drop(ctx, cc.x2); drop(ctx, cc.lse); drop(ctx, cc.xn); drop(ctx, cc.q); drop(ctx, cc.k);
         drop(ctx, cc.v); drop(ctx, cc.attn); drop(ctx, cc.x2n); drop(ctx, cc.h13); drop(ctx, cc.gate);
     }
-    drop(ctx, T->xlast); drop(ctx, T->xf); drop(ctx, T->dlh); drop(ctx, T->dlT); drop(ctx, T->H1); drop(ctx, T->H1m);
+    drop(ctx, T->xlast); drop(ctx, T->xf); drop(ctx, T->dlh); drop(ctx, T->H1); drop(ctx, T->H1m);
     drop(ctx, T->H2); drop(ctx, T->H2q); drop(ctx, T->dOh); drop(ctx, T->gout); drop(ctx, T->dres);
     drop(ctx, T->Drow); drop(ctx, T->dgp); drop(ctx, T->utok); drop(ctx, T->ustart); drop(ctx, T->uidx);
-    for (auto& pr : T->tx)
-        for (f16*& p : pr) drop(ctx, p);
+    drop_copies(ctx);
     const rh_config& c = ctx->cfg;
     const size_t D = c.dim, F = c.hidden, V = c.vocab, Vp = round_up(V, 128);
     const size_t m = M, m16 = round_up(m, 16), mp = round_up(m, 128);
@@ -224,14 +250,10 @@ int ensure_train_ws(rh_ctx* ctx, int B, int S) {
     RCK(dalloc(ctx, &T->xlast, m * D));
     RCK(dalloc(ctx, &T->xf, m16 * D));
     RCK(dalloc(ctx, &T->dlh, m16 * Vp));
-    RCK(dalloc(ctx, &T->dlT, Vp * mp));
     RCK(dalloc(ctx, &T->H1, m16 * D));
     RCK(dalloc(ctx, &T->H1m, m16 * D));
     RCK(dalloc(ctx, &T->H2, m16 * 2 * F));
     RCK(dalloc(ctx, &T->H2q, m16 * 3 * D));
-    const size_t txr[4][2] = {{D, F}, {D, 2 * F}, {D, D}, {D, 3 * D}};  // rows of each copy
-    for (int g = 0; g < 4; ++g)
-        for (int i = 0; i < 2; ++i) RCK(dalloc(ctx, &T->tx[g][i], txr[g][i] * mp));
     RCK(dalloc(ctx, &T->dOh, m * D));
     RCK(dalloc(ctx, &T->gout, m * D));  // an unsplit data-gradient product [M][D]
     RCK(dalloc(ctx, &T->dres, m * D));
@@ -359,11 +381,10 @@ int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float
 // at K = 4096, dWq..dWv 85 -> 32 us, dW1 dW3 62 -> 50; 4096 wide three products
 // of one round each stay (334 against 358 us).  Outputs whose first store the
 // store-wave kernel takes stay n products up to 512 tokens, where writing them
-// is most of the time: forward + backward of two layers after a zero, 128 / 256
-// / 512 tokens, joint -> n products, us: 2560 wide 864 -> 854, 979 -> 961, 1228
-// -> 1210, 3072 wide 1009 -> 995, 1127 -> 1112, 1522 -> 1494, 5120 wide 1775 ->
-// 1702, 2162 -> 2096, 3036 -> 3069 (1024 tokens: 1846 -> 1857, 2242 -> 2212 and
-// 4954 -> 5180).
+// is most of the time: forward + backward of two layers after a zero, joint ->
+// n products, 128 - 512 tokens: 2560 wide 0 - 2% faster, 3072 wide 1 - 4% (512
+// tokens 1510 -> 1455 us), 5120 wide 6% (128 tokens, 1750 -> 1652 us) to -1%
+// (512); at 1024 tokens 3072 wide 1% faster, 5120 wide 4% slower.
 int grad_gemms(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* const* out, int n,
                hipStream_t st, int trx = 0, int trw = 0) {
     if (n == 1 || (ctx->train->Mp <= 512 && store_waves(ctx, rows, cols)) ||
@@ -866,6 +887,7 @@ int prepare_train(rh_ctx* ctx, const uint32_t* tokens, const uint32_t* targets, 
     RCK(ensure_rope(ctx, seq));
     RCK(ensure_train_static(ctx));
     RCK(ensure_train_ws(ctx, batch, seq));
+    RCK(ensure_copies(ctx));
     RCK(ensure_packs(ctx));
     return RH_OK;
 }

@@ -8,6 +8,7 @@ import numpy as np
 import pytest
 
 from rustane_amd import hip_bridge as hb
+from rustane_amd import hip_rt
 from rustane_amd.engine import ModelWeights
 
 from helpers import LOGIT_ATOL, random_gammas, small_cfg, tokens_uniform
@@ -265,3 +266,39 @@ def test_weight_gradients_of_whole_blocks(orc, heads, hidden, nlayers, batch, se
     w = random_gammas(ModelWeights.normal(cfg, seed=370 + heads, std=0.05), 371)
     tok, tgt = tokens_uniform(372 + seq, cfg.vocab, batch, cfg.seq)
     _run(orc, cfg, w, tok, tgt, calls=calls)
+
+
+def test_operand_copies_come_with_the_first_ragged_call():
+    """The transposed operand copies are allocated by the first token count
+    that is no multiple of 128, once, for the largest count seen; calls before
+    and after it give the same bits as in a context of their own."""
+    cfg = small_cfg(dim=512, hidden=1408, heads=8, hd=64, nlayers=1, vocab=32000, seq=1024)
+    copies = (32000 + 8 * 512 + 3 * 1408) * 2048 * 2
+    whole, ragged = tokens_uniform(380, cfg.vocab, 2, 1024), tokens_uniform(381, cfg.vocab, 2, 1000)
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip_rt.rt().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    def grads(c, batch):
+        c.zero_grads()
+        c.forward_backward(*batch, 256.0)
+        g = c.read_grads()
+        return [g[0], g[1], *g[2][0]]
+
+    def same(a, b):
+        return all(np.array_equal(x, y) for x, y in zip(a, b))
+
+    with hb.Context(cfg.to_rh(), 0, 2, 0) as c:
+        c.init_normal(382, 0.02)
+        want_ragged = grads(c, ragged)
+    with hb.Context(cfg.to_rh(), 0, 2, 0) as c:
+        c.init_normal(382, 0.02)
+        want_whole = grads(c, whole)
+        before = free()
+        assert same(grads(c, whole), want_whole) and free() == before
+        assert same(grads(c, ragged), want_ragged)
+        after = free()
+        assert before - after >= copies
+        assert same(grads(c, ragged), want_ragged) and same(grads(c, whole), want_whole) and free() == after
