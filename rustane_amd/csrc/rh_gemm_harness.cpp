@@ -200,8 +200,8 @@ int rhh_gemm_wgrad(const uint16_t* wf, const uint16_t* xf, int M, int N, int K, 
 // 0..M-1 and W's w_off..w_off+N-1 (w_off a multiple of 32); 0: row-major
 // operands as above.  part_cols > 0: the N features go to up to three outputs
 // [M][part_cols] (io0, io1, io2), else to io0 [M][N].  accumulate: io += alpha
-// * product, else io = alpha * product.  cfg: a GemmCfg value, 0 (the tile
-// model) or -1 (the store-wave kernel: one output, no accumulation).
+// * product, else io = alpha * product.  cfg: a GemmCfg value or 0 (the tile
+// model).
 int rhh_gemm_grads(int cfg, int accumulate, const uint16_t* wf, const uint16_t* xf, int M, int N, int K, int trx,
                    int trw, int w_off, float alpha, int part_cols, float* io0, float* io1, float* io2) {
     if (M <= 0 || N <= 0 || K <= 0 || !wf || !xf || !io0 || w_off < 0 || w_off % 32) return -1;
@@ -210,7 +210,6 @@ int rhh_gemm_grads(int cfg, int accumulate, const uint16_t* wf, const uint16_t* 
     if (part_cols ? part_cols < 0 || N > 3 * part_cols || (N > part_cols && !io1) || (N > 2 * part_cols && !io2)
                   : io1 || io2)
         return -1;
-    if (cfg < 0 && (part_cols || accumulate)) return -1;
     Dev d;
     const size_t wn = tr ? (size_t)K * trw : (size_t)up16(N) * K, xn = tr ? (size_t)K * trx : (size_t)up16(M) * K;
     const int cols = part_cols ? part_cols : N;
@@ -232,9 +231,8 @@ int rhh_gemm_grads(int cfg, int accumulate, const uint16_t* wf, const uint16_t* 
     a.trx = trx; a.trw = trw;
     a.out_f32 = out[0]; a.out_part1 = out[1]; a.out_part2 = out[2];
     a.part_cols = part_cols; a.ldo = cols; a.alpha = alpha; a.nt_out = true;
-    a.force_cfg = cfg > 0 ? cfg : 0;
-    hipError_t e = cfg < 0 ? rh::launch_gemm_wgrad(a, false, nullptr)
-                           : rh::launch_gemm(accumulate ? rh::EPI_RESID : rh::EPI_F32, a, nullptr);
+    a.force_cfg = cfg;
+    hipError_t e = rh::launch_gemm(accumulate ? rh::EPI_RESID : rh::EPI_F32, a, nullptr);
     if (e != hipSuccess) return (int)e;
     if ((e = hipDeviceSynchronize()) != hipSuccess) return (int)e;
     for (int i = 0; i < 3; ++i)

@@ -41,8 +41,8 @@ struct GemmArgs {
     // to three outputs [M][ldo = part_cols]: out_f32, out_part1, out_part2.
     int part_cols;
     float *out_part1, *out_part2;
-    // EPI_F32 / EPI_RESID and the weight-gradient kernel: trx, trw > 0 when X
-    // and W are token-major, X [K][trx] and W [K][trw] in fragment order (K
+    // EPI_F32 / EPI_RESID of launch_gemm: trx, trw > 0 when X and W are
+    // token-major, X [K][trx] and W [K][trw] in fragment order (K
     // tokens; all three multiples of 128), read as their transposes.  W may
     // point at feature f (a multiple of 32) of its rows, 16 f halves further,
     // where N features from f on lie within the row.
@@ -111,8 +111,8 @@ hipError_t launch_gemm_partials(const GemmArgs& a, int* nsplit, hipStream_t st);
 // Weight-gradient GEMM for a short K (the token count): out [M][ldo] fp32 =
 // alpha * X W^T (alpha 0: unscaled), or += when accumulate; persistent blocks
 // whose store waves write each 128x128 tile while the next one is computed.
-// Needs K % 128 == 0, N % 4 == 0.  The backward only stores; token-major
-// operands (trx, trw) are not built to accumulate.
+// Needs K % 128 == 0, N % 4 == 0 and row-major operands.  The backward only
+// stores.
 hipError_t launch_gemm_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st);
 
 // ---------------- attention ----------------

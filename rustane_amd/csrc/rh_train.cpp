@@ -18,10 +18,11 @@
 // Every product is an NT GEMM of the forward's kernel: the data-gradient
 // GEMMs stream transposed copies of the weights (built once per weight
 // version), the weight-gradient GEMMs contract over tokens (whole blocks of
-// 128 read in place by transposing LDS reads, ragged counts from token-inner
-// copies of the operands), and accumulate into the
-// fp32 gradients in their epilogue (C += kappa * acc).  Gradients keep the
-// reference's tensor shapes and orientation and accumulate across calls.
+// 128 read in place by transposing LDS reads; ragged counts, and short first
+// stores of large outputs, from token-inner copies of the operands), and
+// accumulate into the fp32 gradients in their epilogue (C += kappa * acc).
+// Gradients keep the reference's tensor shapes and orientation and accumulate
+// across calls.
 #include "rh_ctx.h"
 
 #include <algorithm>
@@ -61,7 +62,7 @@ struct TrainState {
     f16 *dlh = nullptr, *H1 = nullptr, *H1m = nullptr, *H2 = nullptr, *H2q = nullptr;
     // The weight-gradient GEMMs run on the side stream in four groups per
     // layer (0: dW2, 1: dW1 dW3, 2: dWo, 3: dWq dWk dWv), from the activation
-    // gradient above and a forward cache, or for ragged token counts from
+    // gradient above and a forward cache, or (enqueue_backward says when) from
     // token-inner copies of them, tx[g] and dlT (written on the side stream too).
     // ready[g] (main): group g's activation gradient is written; read[g]
     // (side): it has been read (by the GEMM, or by the copy), so the main
@@ -182,6 +183,15 @@ int ensure_train_static(rh_ctx* ctx) {
     return RH_OK;
 }
 
+// Whether the store-wave kernel takes the first store of a gradient [rows][cols]
+// (store_waves: of this call's).
+bool store_wave_size(const rh_ctx* ctx, size_t rows, size_t cols) {
+    return ctx->train->Mp <= 1024 && rows * cols >= (size_t)4096 * 4096;
+}
+bool store_waves(const rh_ctx* ctx, int rows, int cols) {
+    return ctx->train->zero && store_wave_size(ctx, rows, cols);
+}
+
 void drop_copies(rh_ctx* ctx) {
     TrainState* T = ctx->train;
     T->txM = 0;
@@ -190,12 +200,15 @@ void drop_copies(rh_ctx* ctx) {
         for (f16*& p : pr) drop(ctx, p);
 }
 
-// The token-inner copies, which only token counts that are no multiple of 128
-// need (0.8 GB at 4096 wide, vocabulary 32000 and 4096 tokens): sized for the
-// buffers' capacity by the first such call.
+// The token-inner copies (0.8 GB at 4096 wide, vocabulary 32000 and 4096
+// tokens), sized for the buffers' capacity by the first call that needs them:
+// a token count that is no multiple of 128, or outputs that the store-wave
+// kernel takes when they are next zeroed.
 int ensure_copies(rh_ctx* ctx) {
     TrainState* T = ctx->train;
-    if (T->B * T->S == T->Mp || T->txM >= T->M) return RH_OK;
+    const size_t d = ctx->cfg.dim, f = ctx->cfg.hidden, v = ctx->cfg.vocab;
+    const bool need = T->B * T->S != T->Mp || store_wave_size(ctx, d, std::max({d, f, v}));
+    if (!need || T->txM >= T->M) return RH_OK;
     HCK(hipStreamSynchronize(T->side));  // reads them
     drop_copies(ctx);
     const rh_config& c = ctx->cfg;
@@ -344,11 +357,6 @@ int gamma_grad(rh_ctx* ctx, int nblk, int D, float kappa, float* dgamma) {
     return RH_OK;
 }
 
-// Whether the store-wave kernel takes the first store of a gradient [rows][cols].
-bool store_waves(const rh_ctx* ctx, int rows, int cols) {
-    return ctx->train->zero && ctx->train->Mp <= 1024 && (size_t)rows * cols >= (size_t)4096 * 4096;
-}
-
 // C[rows][cols] += kappa * X W^T with X [rows][Mp], W [cols][Mp] (token-inner).
 // When every gradient is still zero the epilogue stores kappa * acc instead
 // (the same values; it skips reading the fp32 gradient back).  The tile model
@@ -375,20 +383,24 @@ int grad_gemm(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float
     return RH_OK;
 }
 
-// n (2 or 3) gradients [rows][cols] of one X, the W of each after the other:
-// dWq | dWk | dWv and dW1 | dW3.  As one product with n outputs where that
-// fills the CUs better than n products (the tile model's estimate): 1024 wide
-// at K = 4096, dWq..dWv 85 -> 32 us, dW1 dW3 62 -> 50; 4096 wide three products
+// Whether n (2 or 3) gradients [rows][cols] of one X (dWq | dWk | dWv and dW1 |
+// dW3) run as one product with n outputs: where that fills the CUs better than
+// n products (the tile model's estimate): 1024 wide at K = 4096, dWq..dWv 85 -> 32 us, dW1 dW3 62 -> 50; 4096 wide three products
 // of one round each stay (334 against 358 us).  Outputs whose first store the
 // store-wave kernel takes stay n products up to 512 tokens, where writing them
 // is most of the time: forward + backward of two layers after a zero, joint ->
 // n products, 128 - 512 tokens: 2560 wide 0 - 2% faster, 3072 wide 1 - 4% (512
 // tokens 1510 -> 1455 us), 5120 wide 6% (128 tokens, 1750 -> 1652 us) to -1%
 // (512); at 1024 tokens 3072 wide 1% faster, 5120 wide 4% slower.
+bool joint(const rh_ctx* ctx, int rows, int cols, int n) {
+    if (n == 1 || (ctx->train->Mp <= 512 && store_waves(ctx, rows, cols))) return false;
+    return rh::gemm_tile_cost(rows, n * cols) < (float)n * rh::gemm_tile_cost(rows, cols);
+}
+
+// n gradients [rows][cols] of one X, the W of each after the other.
 int grad_gemms(rh_ctx* ctx, const f16* X, const f16* W, int rows, int cols, float kappa, float* const* out, int n,
                hipStream_t st, int trx = 0, int trw = 0) {
-    if (n == 1 || (ctx->train->Mp <= 512 && store_waves(ctx, rows, cols)) ||
-        rh::gemm_tile_cost(rows, n * cols) >= (float)n * rh::gemm_tile_cost(rows, cols)) {
+    if (!joint(ctx, rows, cols, n)) {
         for (int j = 0; j < n; ++j)
             RCK(grad_gemm(ctx, X, W + (size_t)j * cols * (trw ? 16 : ctx->train->Mp), rows, cols, kappa, out[j], st,
                           trx, trw));
@@ -455,27 +467,32 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
     LCK(rh::launch_ce_backward(ctx->logits, ctx->d_tgt, T->dlh, M, V, Vp, T->fwd_softcap, rh::GRAD_UNIT, st));
     RCK(publish(4));
     // Weight gradients contract over tokens.  With whole 128-token blocks the
-    // GEMMs read the token-major activations and their gradients in place
-    // (then read[g] is the GEMM's end), which was 0.3 - 12% faster at every
-    // width (512 - 4096) and token count (128 - 8192) timed; otherwise the rows
-    // past the last token have to be zeros and they take padded token-inner
-    // copies.
-    const bool tr = M == Mp;
-    auto grads = [&](int g, const f16* X, int nx, const f16* W, int nw, int rows, int cols, float* const* out,
-                     int n) -> int {
+    // tile kernels read the token-major activations and their gradients in place
+    // (then read[g] is the GEMM's end); otherwise the rows past the last token
+    // have to be zeros and the GEMMs take padded token-inner copies.  From 1000
+    // tokens on that is 1 - 6% of a pass at every width (512 - 4096; 20 layers of
+    // 4096, 8 x 512 accumulated: 98.2 -> 95.3 ms), at 128 - 512 tokens 7% (2304
+    // wide) to -5% (512 wide).  The store-wave kernel keeps the copies: two
+    // transposing reads for each of its 128x128 tile's operands take 4096 x
+    // 11008 x 512 from 72 to 93 us beside the other stream (20 layers of 4096
+    // after a zero, 1 x 512: 19.7 ms in place, 18.7 with copies).
+    auto in_place = [&](int rows, int cols, int n) {
+        return M == Mp && (joint(ctx, rows, cols, n) || !store_waves(ctx, rows, cols));
+    };
+    auto grads = [&](int g, const f16* X, int nx, f16* Xt, const f16* W, int nw, f16* Wt, int rows, int cols,
+                     float* const* out, int n) -> int {
+        const bool tr = in_place(rows, cols, n);
         if (!tr) {
-            LCK(rh::launch_transpose_frag2(X, T->tx[g][0], M, nx, W, T->tx[g][1], M, nw, Mp, sd));
-            HCK(hipEventRecord(T->read[g], sd));
-            X = T->tx[g][0];
-            W = T->tx[g][1];
+            LCK(rh::launch_transpose_frag2(X, Xt, M, nx, W, Wt, M, nw, Mp, sd));
+            if (g >= 0) HCK(hipEventRecord(T->read[g], sd));
+            X = Xt;
+            W = Wt;
         }
         RCK(grad_gemms(ctx, X, W, rows, cols, kappa, out, n, sd, tr ? nx : 0, tr ? nw : 0));
-        if (tr) HCK(hipEventRecord(T->read[g], sd));
+        if (tr && g >= 0) HCK(hipEventRecord(T->read[g], sd));
         return RH_OK;
     };
-    if (!tr) LCK(rh::launch_transpose_frag2(T->dlh, T->dlT, M, Vp, T->xf, T->tx[0][0], M, D, Mp, sd));
-    RCK(grad_gemm(ctx, tr ? T->dlh : T->dlT, tr ? T->xf : T->tx[0][0], V, D, kappa, T->dembed, sd, tr ? Vp : 0,
-                  tr ? D : 0));
+    RCK(grads(-1, T->dlh, Vp, T->dlT, T->xf, D, T->tx[0][0], V, D, &T->dembed, 1));
     const size_t MD = (size_t)M * D;  // stride of the data-gradient partials
     const float* dp;
     int ns;
@@ -491,7 +508,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         float* const* G = T->dlay[l].data();
         // dW2 += dffn^T gate (side); dgate = dffn W2 with the SiLU backward -> [dh1 | dh3]
         RCK(publish(0));
-        RCK(grads(0, T->H1, D, cc.gate, F, D, F, G + 6, 1));
+        RCK(grads(0, T->H1, D, T->tx[0][0], cc.gate, F, T->tx[0][1], D, F, G + 6, 1));
         RCK(rewrite(1));
         {
             rh::GemmArgs g{};
@@ -502,7 +519,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         }
         // dx_ffn = [dh1 | dh3] [W1 | W3]^T; dW1, dW3 += x2n^T dh (side)
         RCK(publish(1));
-        RCK(grads(1, cc.x2n, D, T->H2, 2 * F, D, F, G + 4, 2));
+        RCK(grads(1, cc.x2n, D, T->tx[1][0], T->H2, 2 * F, T->tx[1][1], D, F, G + 4, 2));
         RCK(data_gemm(ctx, T->H2, wt.w13t, M, D, 2 * F, T->gout, &dp, &ns));
         // dx2 = RMSNorm2'(dx_ffn) + dy (in place in dres); a*dx2 -> H1m
         RCK(rewrite(2));
@@ -511,7 +528,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
         RCK(gamma_grad(ctx, nblk, D, kappa, G[8]));
         // da = (a dx2) Wo^T; dWo += attn^T (a dx2) (side)
         RCK(publish(2));
-        RCK(grads(2, cc.attn, D, T->H1m, D, D, D, G + 3, 1));
+        RCK(grads(2, cc.attn, D, T->tx[2][0], T->H1m, D, T->tx[2][1], D, D, G + 3, 1));
         RCK(data_gemm(ctx, T->H1m, wt.ot, M, D, D, T->gout, &dp, &ns));
         // attention backward -> dq | dk | dv with the RoPE backward, as the fp16
         // operand H2q (rewritten: the side stream has copied the previous layer's)
@@ -520,7 +537,7 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
                                      ctx->rope, B, H, S, hd, st));
         // dxn = dqkv [Wq | Wk | Wv]^T; dWq, dWk, dWv += xn^T d{q,k,v} (side)
         RCK(publish(3));
-        RCK(grads(3, cc.xn, D, T->H2q, 3 * D, D, D, G, 3));
+        RCK(grads(3, cc.xn, D, T->tx[3][0], T->H2q, 3 * D, T->tx[3][1], D, D, G, 3));
         RCK(data_gemm(ctx, T->H2q, wt.qkvt, M, D, 3 * D, T->gout, &dp, &ns));
         // dy' = RMSNorm1'(dxn) + dx2 (in place); a*dy' -> H1 (the next layer's dffn)
         RCK(rewrite(0));

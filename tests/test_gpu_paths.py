@@ -148,10 +148,11 @@ def test_joint_weight_gradients(orc, heads, hidden, calls):
 
 
 # 2560 x 6912: up to 512 tokens the first dW1 and dW3 are two products of the
-# store-wave kernel, later ones (and longer first ones) one product with two
-# outputs.  Both sum the tokens in order, and with powers of two for the loss
-# scale and the length every scaling is exact: a second call on the same batch
-# doubles the gradients to the bit.
+# store-wave kernel on transposed copies, later ones (and longer first ones) one
+# product with two outputs, in place.  All sum the tokens in order, and with
+# powers of two for the loss scale and the length every scaling is exact: a
+# second call on the same batch doubles the gradients to the bit, and a zero
+# between a forward and its backward gives the first ones again.
 @pytest.mark.parametrize("seq", [128, 256, 512, 1024])
 def test_first_and_joint_weight_gradients_agree(seq):
     cfg = small_cfg(dim=2560, hidden=6912, heads=20, hd=128, nlayers=1, vocab=512, seq=seq)
@@ -162,8 +163,12 @@ def test_first_and_joint_weight_gradients_agree(seq):
         first = c.read_grads()[2][0]
         c.forward_backward(tok, tgt, 256.0)
         second = c.read_grads()[2][0]
+        fwd, _ = c.forward_train(tok, tgt)
+        c.zero_grads()
+        c.backward(fwd, loss_scale=256.0)
+        third = c.read_grads()[2][0]
     for j in range(7):
-        assert first[j].any() and np.array_equal(second[j], 2 * first[j]), j
+        assert first[j].any() and np.array_equal(second[j], 2 * first[j]) and np.array_equal(third[j], first[j]), j
 
 
 def grads_product(lib, cfg, accumulate, x, w, M, N, alpha, outs, part_cols=0, w_off=0, tokens=False):  # noqa: F811
@@ -182,25 +187,23 @@ PICKED = ["D8_256x256", "D8_256x128", "D8_192x256", "D8_192x128", "D8_128x128"] 
 
 
 # Products over tokens with both operands token-major, every tile the model can
-# pick and the store-wave kernel: outputs that end inside a tile and inside a
-# 32-feature block, operand rows wider than the product and a W that starts
-# inside its rows (dW3's), k loops shorter than the stage rings and ending on
-# each of their buffers, and more tiles than blocks or groups of 8 M-tiles.
+# pick: outputs that end inside a tile and inside a 32-feature block, operand
+# rows wider than the product and a W that starts inside its rows (dW3's), k
+# loops shorter than the stage rings and ending on each of their buffers, and
+# more tiles than CUs or groups of 8 M-tiles.
 # fp32 sums of K <= 640 products: 1e-5 of max|Y|.
 @pytest.mark.parametrize("M,N,K,trx,trw,w_off", [(4, 4, 128, 128, 128, 0), (600, 700, 128, 640, 768, 32),
                                                  (300, 1000, 256, 384, 1152, 96), (600, 700, 384, 640, 768, 64),
                                                  (300, 516, 640, 384, 640, 0), (2100, 2200, 128, 2176, 2304, 0)])
-@pytest.mark.parametrize("name", PICKED + ["store_waves"])
+@pytest.mark.parametrize("name", PICKED)
 def test_products_over_tokens(lib, name, M, N, K, trx, trw, w_off):  # noqa: F811
     rng = np.random.default_rng(28)
     x, w = (rng.standard_normal((K, n)).astype(np.float16) for n in (trx, trw))
     y = x[:, :M].T.astype(np.float64) @ w[:, w_off:w_off + N].astype(np.float64)
-    cfg = CFGS.get(name, -1)
+    cfg = CFGS[name]
     out = np.full((M, N), np.nan, np.float32)
     grads_product(lib, cfg, 0, x, w, M, N, 0.5, [out], w_off=w_off, tokens=True)
     close(out, 0.5 * y, 1e-5, f"{name} store")
-    if cfg < 0:
-        return
     x0 = rng.standard_normal((M, N)).astype(np.float32)
     io = x0.copy()
     grads_product(lib, cfg, 1, x, w, M, N, 0.25, [io], w_off=w_off, tokens=True)
@@ -228,7 +231,8 @@ def test_products_with_several_outputs(lib, name, part_cols, N, tokens):  # noqa
         got = np.concatenate(outs, 1)
         before = np.concatenate(list(old), 1)
         assert np.array_equal(got[:, N:], before[:, N:])
-        close(got[:, :N], before[:, :N].astype(np.float64) * accumulate + 0.5 * y, 1e-5, f"{name} accumulate {accumulate}")
+        want = before[:, :N].astype(np.float64) * accumulate + 0.5 * y
+        close(got[:, :N], want, 1e-5, f"{name} accumulate {accumulate}")
 
 
 # Attention backward at head dim 128: lengths that end inside and on a 64-row
@@ -254,10 +258,10 @@ def test_rmsnorm_backward_widths(orc, heads, hd, seq):
 
 
 # Weight gradients of whole 128-token blocks read the token-major operands in
-# place, others take transposed copies: token counts on both sides, one and
-# several layers (each buffer rewritten a layer after its product read it), a
-# vocabulary that ends inside a tile, and (8, 2816), whose dW1 | dW3 runs on
-# 192-wide tiles that straddle the outputs.
+# place (at these sizes), others take transposed copies: token counts on both
+# sides, one and several layers (each buffer rewritten a layer after its product
+# read it), a vocabulary that ends inside a tile, and (8, 2816), whose dW1 | dW3
+# runs on 192-wide tiles that straddle the outputs.
 @pytest.mark.parametrize("heads,hidden,nlayers", [(1, 128, 1), (3, 640, 2), (5, 1408, 3), (8, 2816, 1)])
 @pytest.mark.parametrize("batch,seq", [(1, 128), (2, 64), (3, 128), (2, 96)])
 @pytest.mark.parametrize("calls", [1, 2])
