@@ -32,6 +32,18 @@ def test_embedding_gradient_of_repeated_tokens(orc):
     _run(orc, cfg, w, np.ascontiguousarray(tok), tgt)
 
 
+@pytest.mark.parametrize("vocab,ids", [(128, [0, 127]), (2048, [0, 1, 1024, 2047]), (2052, [3, 2047, 2048, 2051]),
+                                       (6152, [0, 1, 2047, 2048, 2049, 4095, 4096, 4097, 6144, 6151])])
+def test_embedding_gradient_index(orc, vocab, ids):
+    """Ids on either side of the index's 11-bit sort digits, equal in one digit
+    and not in the other, and a vocabulary that one pass covers."""
+    cfg = small_cfg(dim=128, hidden=128, heads=1, hd=128, nlayers=1, vocab=vocab, seq=40)
+    w = random_gammas(ModelWeights.normal(cfg, seed=304, std=0.05), 305)
+    rng = np.random.default_rng(306)
+    tok = rng.choice(np.array(ids, np.uint32), size=(2, 40))
+    _run(orc, cfg, w, tok, rng.integers(0, vocab, size=tok.shape).astype(np.uint32))
+
+
 @pytest.mark.parametrize("K", [128, 256, 384, 640, 1152])
 @pytest.mark.parametrize("name", ["D8_256x256", "D8_256x256_SK", "D8_256x128", "D8_256x128_SK"])
 def test_ping_pong_step_counts(lib, name, K):  # noqa: F811
