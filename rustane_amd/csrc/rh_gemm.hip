@@ -930,7 +930,7 @@ template <int EPI>
 hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
     int cfg = a.force_cfg;
     if constexpr (EPI == EPI_F32 || EPI == EPI_SWIGLU || EPI == EPI_QKV) {
-        if (cfg == GCFG_AUTO && a.M <= SKINNY_M) return launch_gemm_skinny(EPI, a, st);
+        if (cfg == GCFG_AUTO && skinny_takes(EPI, a)) return launch_gemm_skinny(EPI, a, st);
     }
     if (cfg == GCFG_AUTO) {
         const long long KT = a.K / 32;

@@ -84,6 +84,9 @@ enum GemmCfg {
 // 7B prefill takes 4.52 -> 3.62 ms at 64 tokens (past them a fifth token tile
 // would not leave room for the weights in flight; tile kernels 4.58 ms at 65).
 constexpr int SKINNY_M = 64;
+// Whether launch_gemm_skinny takes the product (W1|W3 of some widths only up to
+// 32 tokens).
+bool skinny_takes(int epi, const GemmArgs& a);
 int skinny_splits(const GemmArgs& a);
 hipError_t launch_gemm_skinny(int epi, const GemmArgs& a, hipStream_t st);
 hipError_t launch_gemm_skinny_split(const GemmArgs& a, int S, hipStream_t st);

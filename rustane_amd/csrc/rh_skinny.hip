@@ -21,8 +21,9 @@
 // kernel sums the partials).
 //
 // Measured (us, tile kernel -> this, weights from HBM): 7B, 45 tokens: QKV 36
-// (stream-K and fix-up) -> 21, W1|W3 45 -> 35, W2 26 -> 19, Wo 8.7 -> 9.3; 600M:
-// QKV 13.5 -> 7.1, W1|W3 11.8 -> 7.9, W2 6.6 -> 5.5, Wo 5.0 -> 3.9.
+// (stream-K and fix-up) -> 21, W1|W3 45 -> 35, W2 26 -> 19, Wo 8.7 -> 9.3 (half
+// as many splits for its row kernel to read); 600M: QKV 13.5 -> 7.1, W1|W3 11.8 ->
+// 7.9, W2 6.6 -> 5.5, Wo 5.0 -> 3.9.
 #include <algorithm>
 
 #include <hip/hip_ext.h>
@@ -140,12 +141,15 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(GemmArgs a, int S) {
     }
 }
 
-template <int EPI, int RT, bool SPLIT>
+// MTM: the most token tiles there is a kernel for.
+template <int EPI, int RT, bool SPLIT, int MTM = 4>
 hipError_t launch_rt(const GemmArgs& a, int S, hipStream_t st) {
     const dim3 grid((a.N + 16 * RT - 1) / (16 * RT) * S), blk(512);
 #define RH_SKN(MT_)                                                                                              \
     case MT_:                                                                                                    \
-        if (a.prof_start)                                                                                        \
+        if constexpr (MT_ > MTM)                                                                                 \
+            return hipErrorInvalidValue;                                                                         \
+        else if (a.prof_start)                                                                                   \
             hipExtLaunchKernelGGL((gemm_skinny_kernel<EPI, RT, MT_, SPLIT>), grid, blk, 0, st, a.prof_start,     \
                                   a.prof_stop, 0u, a, S);                                                        \
         else                                                                                                     \
@@ -159,9 +163,17 @@ hipError_t launch_rt(const GemmArgs& a, int S, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Row tiles per block of the split form, and its split count: about one
-// block per CU, at most 8 splits.
-int split_rt(int N) { return N >= 2560 ? 4 : 2; }
+// Row tiles per block with one block per CU.
+int row_tiles_per_cu(int N) { return ((N + 15) / 16 + 255) / 256; }
+
+// Row tiles per block of the split form (about one block per CU, at most 8
+// splits): 4, or 2 for narrow outputs.  3 where that gives as many splits (of
+// the outputs that split, N 5441 - 6144: with 4 a third of the CUs had no block).
+int split_rt(int N) {
+    const int nrt = (N + 15) / 16;
+    if (N < 2560) return 2;
+    return 256 / ((nrt + 2) / 3) == 256 / ((nrt + 3) / 4) ? 3 : 4;
+}
 
 }  // namespace
 
@@ -177,17 +189,40 @@ hipError_t launch_gemm_skinny_split(const GemmArgs& a, int S, hipStream_t st) {
     if (a.M <= 0 || a.M > SKINNY_M || a.K % 128 != 0 || a.N % 4 != 0 || S < 1 || S > a.K / 128 || !a.sk_part ||
         (size_t)S * a.M * a.N > a.sk_part_floats)
         return hipErrorInvalidValue;
-    return split_rt(a.N) == 4 ? launch_rt<EPI_F32, 4, true>(a, S, st) : launch_rt<EPI_F32, 2, true>(a, S, st);
+    switch (split_rt(a.N)) {
+        case 4: return launch_rt<EPI_F32, 4, true>(a, S, st);
+        case 3: return launch_rt<EPI_F32, 3, true>(a, S, st);
+    }
+    return launch_rt<EPI_F32, 2, true>(a, S, st);
+}
+
+// The row tiles per block follow the width so that one round of blocks covers the
+// rows: QKV takes 6 at 8192 wide, W1|W3 8 at 5632 wide (15104 hidden features).
+// With at most 4 and 6 the blocks past 256 ran a second round.  16 | 64 tokens, us,
+// tile kernel -> at most 4 and 6 -> as here: QKV 5632 wide 52 -> 44 -> 33 | 54 -> 60
+// -> 42, 8192 wide 93 -> 71 -> 64 | 94 -> 89 -> 71; W1|W3 4608 wide 48 -> 54 -> 40 |
+// 52 -> 64 -> 46, 5120 wide 55 -> 63 -> 49 | 61 -> 76 -> 52.
+// 8 row tiles of more than 32 tokens do not fit the registers; there the tile
+// kernel stays.  Wider W1|W3 run 6 row tiles in two rounds: 6144 wide 86 -> 77 | 95
+// -> 91, 8192 wide 134 -> 109 | 130 -> 125 (of the widths timed only 7680 at 64
+// tokens loses, 110 -> 120, beside 76 -> 65 of its QKV).
+bool skinny_takes(int epi, const GemmArgs& a) {
+    if (a.M > SKINNY_M) return false;
+    const int per = row_tiles_per_cu(a.N);
+    return !(epi == EPI_SWIGLU && (per == 7 || per == 8) && a.M > 32);
 }
 
 hipError_t launch_gemm_skinny(int epi, const GemmArgs& a, hipStream_t st) {
     if (a.M <= 0 || a.M > SKINNY_M || a.K % 128 != 0 || a.N % 4 != 0) return hipErrorInvalidValue;
-    const int per = ((a.N + 15) / 16 + 255) / 256;  // row tiles per block with one block per CU
+    const int per = row_tiles_per_cu(a.N);
     switch (epi) {
         case EPI_QKV:
-            if (per >= 4) return launch_rt<EPI_QKV, 4, false>(a, 1, st);
+            if (per >= 6) return launch_rt<EPI_QKV, 6, false>(a, 1, st);
+            if (per == 5) return launch_rt<EPI_QKV, 5, false>(a, 1, st);
+            if (per == 4) return launch_rt<EPI_QKV, 4, false>(a, 1, st);
             return per == 3 ? launch_rt<EPI_QKV, 3, false>(a, 1, st) : launch_rt<EPI_QKV, 2, false>(a, 1, st);
         case EPI_SWIGLU:
+            if (per == 7 || per == 8) return launch_rt<EPI_SWIGLU, 8, false, 2>(a, 1, st);
             if (per >= 5) return launch_rt<EPI_SWIGLU, 6, false>(a, 1, st);
             return per >= 3 ? launch_rt<EPI_SWIGLU, 4, false>(a, 1, st) : launch_rt<EPI_SWIGLU, 2, false>(a, 1, st);
         case EPI_F32:

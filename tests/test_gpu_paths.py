@@ -114,6 +114,25 @@ def test_few_tokens_residual_then_rmsnorm(lib, M, N, K):  # noqa: F811
     close(frag_unpack(xn, M, N), x1 / np.sqrt((x1 * x1).mean(1, keepdims=True) + eps) * gamma, 2e-3, "rmsnorm")
 
 
+# The row tiles per block of wide models: QKV 5 and 6, W1 | W3 8 (up to 32
+# tokens; past them the tile kernel), 6 past 2048 row tiles, the split form 3.
+@pytest.mark.parametrize("B,S,H", [(1, 64, 43), (1, 7, 43), (2, 24, 53), (1, 33, 54), (1, 64, 64)])
+def test_few_tokens_qkv_wide(lib, B, S, H):  # noqa: F811
+    test_few_tokens_qkv(lib, B, S, H, 128)
+
+
+@pytest.mark.parametrize("M", [1, 17, 32, 33, 64])
+@pytest.mark.parametrize("F", [12416, 16384, 16512])
+def test_few_tokens_swiglu_wide(lib, M, F):  # noqa: F811
+    test_few_tokens_swiglu(lib, M, F, 384)
+
+
+@pytest.mark.parametrize("M", [1, 33, 64])
+@pytest.mark.parametrize("N,K", [(5504, 256), (6144, 1408), (6272, 256)])
+def test_few_tokens_residual_then_rmsnorm_wide(lib, M, N, K):  # noqa: F811
+    test_few_tokens_residual_then_rmsnorm(lib, M, N, K)
+
+
 def _decode_matches_forward(cfg, B, p0, steps, seed, max_ctx=0):
     """Teacher-forced decode logits equal the forward's at every position."""
     w = random_gammas(ModelWeights.normal(cfg, seed=seed), seed + 1)
