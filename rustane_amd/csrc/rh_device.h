@@ -107,8 +107,8 @@ __device__ __forceinline__ void lds_barrier() {
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }
 
 // XOR swizzles of the 16-byte chunks of a 256-byte LDS row (an hd-128 fp16
-// K / V / Q / dO row staged by DMA): chunk c of row k is stored at
-// c ^ swz(k).  swz_k keeps the row-fragment reads of a 16x16x32 A operand
+// K or V row of the prefill attention, staged by DMA): chunk c of row k is
+// stored at c ^ swz(k).  swz_k keeps the row-fragment reads of a 16x16x32 A operand
 // (rows 8(r/4) + 4u + r%4, chunk 4kk + g) on distinct banks, swz_v the
 // transposing reads (ds_read_b64_tr_b16) of keys 8g + 4h + r/4.
 __device__ __forceinline__ int swz_k(int row) { return (row & 3) | (((row >> 3) & 3) << 2); }

@@ -896,15 +896,14 @@ __global__ __launch_bounds__(Tl::NT + 64 * WG_SW) void gemm_wgrad_kernel(GemmArg
 }
 
 // Data-parallel tiles: estimated time = rounds of one block per CU x
-// tile FLOPs / that tile's per-CU rate.  The rates are fitted to MI355X
-// timings of every tile on 27 GEMM shapes of the 7B forward and
-// training step (M 512 - 8192, random fp16 operands; the picks land
-// within 0.5% of the per-shape best in total; 256x256 and 256x128 refitted
-// for the ping-pong tiles: at M = 8192 a 256x256 tile takes 1.20 times a
-// 192x256 one's time for 1.33 times its work, at M = 512 1.09 times for a
-// tile of W1|W3); the estimate trades wave
-// quantization (e.g. 172 vs 230 tiles at M = 512) against per-tile
-// efficiency.  Narrow outputs (Wo) and long K (W2) use stream-K
+// tile FLOPs / that tile's per-CU rate.  The rates of 192x256, 192x128 and
+// 128x128 are fitted to MI355X timings of every tile on 27 GEMM shapes of the 7B
+// forward and training step (M 512 - 8192, random fp16 operands), those of
+// 256x256 and 256x128 to the ping-pong tiles: at M = 8192 a 256x256 tile takes
+// 1.20 times a 192x256 one's time for 1.33 times its work, at M = 512 1.09 times
+// for a tile of W1|W3.  The estimate trades wave quantization (e.g. 172 vs 230
+// tiles at M = 512) against per-tile efficiency and knows nothing of the
+// epilogue's bytes, which count at a short K.  Narrow outputs (Wo) and long K (W2) use stream-K
 // instead, when every block gets at least two 32-wide k-iterations.  *cost: the
 // pick's estimate (per unit of K).
 int tile_pick(int M, int N, float* cost) {
@@ -954,9 +953,9 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
     // as a 4-wave 16x16x32 tile and 91.4 as 8-wave 32x32x16; QKV 60.4 us as
     // 8-wave 16x16x32 192x128 against 64.7 as 4-wave 32x32x16; the 8-wave
     // 128x128 tile is 1-6% faster in that form than its 32x32x16 twin on every
-    // shape timed.  8-wave 256x256 and 256x128 are ping-pong tiles.  The
-    // 4-wave 192x128 tile stays 32x32x16 (in the 16x16x32 form its second
-    // block per CU would not fit the registers).
+    // shape timed.  8-wave 256x256 and 256x128 are ping-pong tiles.  The 4-wave
+    // tiles and the stream-K forms that GCFG_AUTO does not name above are taken
+    // only by force_cfg.
     switch (cfg) {
         case GCFG_D8_256x256: return launch_tile<Tile256x256, EPI>(a, false, st);
         case GCFG_D8_256x256_SK: return launch_tile<Tile256x256, EPI>(a, true, st);
@@ -1024,9 +1023,9 @@ hipError_t launch_gemm_wgrad(const GemmArgs& a, bool accumulate, hipStream_t st)
 
 namespace {
 
-// Few tokens: the skinny kernel's own splits.  Else split K when the output has too few tiles to fill the CUs: S splits per
-// tile, at most 8 and at least 8 k-iterations each, within the workspace;
-// 1 = no split.
+// Few tokens: the skinny kernel's own splits.  Else split K when the output has
+// too few tiles to fill the CUs: S splits per tile, at most 8 and at least 8
+// k-iterations each, within the workspace; 1 = no split.
 int split_count(const GemmArgs& a) {
     if (a.force_cfg == GCFG_AUTO && a.M <= SKINNY_M) return skinny_splits(a);
     const int bn = a.K >= 8192 ? 256 : 128, bm = 128;
@@ -1039,11 +1038,10 @@ int split_count(const GemmArgs& a) {
     return S;
 }
 
-// K >= 8192 (W2): 256x128 tiles as 8 waves of 16x16x32 (50.3 vs 52.9 us as 4
-// waves of 32x32x16 at 7B, M = 512; the ping-pong 256x128 tile measures the
-// same there and loses at short prompts, whole 7B prefill of 45 tokens 4.23 ->
-// 4.34 ms); otherwise 128x128 (the two forms measure
-// the same there)
+// Up to SKINNY_M tokens the few-token kernel.  Else K >= 8192 (W2): 256x128
+// tiles as 8 waves of 16x16x32 (50.3 vs 52.9 us as 4 waves of 32x32x16 at 7B,
+// M = 512; the ping-pong 256x128 tile measures the same there); otherwise
+// 128x128 (the two forms measure the same there)
 hipError_t launch_split_any(const GemmArgs& a, int S, hipStream_t st) {
     if (a.M <= SKINNY_M) return launch_gemm_skinny_split(a, S, st);
     return a.K >= 8192 ? launch_split<DTile<4, 2, 2, 2, true>>(a, S, st) : launch_split<DTile<2, 2, 2, 2>>(a, S, st);

@@ -52,9 +52,10 @@ __host__ __device__ constexpr int SXP(int K) { return K + 8; }
 // 2 a wave per token, so that the tokens' round trips overlap instead of
 // following each other through two barriers each (600M, 4 tokens: QKV 10.6 ->
 // 7.6 us, W1|W3 12.3 -> 9.3, logits 32.5 -> 27.8).  A wave walks a long row
-// slower than a block does: whole decode passes at 4096 wide change by -2.4% at
-// 2 tokens, -2.6% at 3 and +2.0% at 4, at 2560 wide by +1.5% at 2, at 1536 by
-// +4.5% at 2 and +24% at 10, at 512 by +42% at 16.  One token keeps the block.
+// slower than a block does: with a wave per token, whole decode passes give 2.4%
+// fewer tokens/s at 4096 wide and 2 tokens, 2.6% fewer at 3 and 2.0% more at 4;
+// at 2560 wide 1.5% more at 2, at 1536 4.5% more at 2 and 24% at 10, at 512 42%
+// more at 16.  One token keeps the block.
 bool norm_by_waves(int B, int K) { return B >= 4 || (B > 1 && K <= 2560); }
 
 template <int EPI, int RT, int NW, int DEPTH, int NORM, bool XF = false>

@@ -53,7 +53,8 @@ struct GemmArgs {
     hipEvent_t prof_start, prof_stop;
 };
 // Tile configurations of the prefill GEMM (all: direct-to-LDS pipeline;
-// waves x per-wave tile).
+// waves x per-wave tile).  GCFG_AUTO takes the 8-wave tiles, 256x128 and 128x128
+// as stream-K too; the others have no caller but the tile tests (force_cfg).
 enum GemmCfg {
     GCFG_AUTO = 0,
     GCFG_D8_256x256 = 6,     // 8 waves (128x64 each), ping-pong, 16x16x32 MFMA
