@@ -903,20 +903,26 @@ __global__ __launch_bounds__(Tl::NT + 64 * WG_SW) void gemm_wgrad_kernel(GemmArg
 // 1.20 times a 192x256 one's time for 1.33 times its work, at M = 512 1.09 times
 // for a tile of W1|W3.  The estimate trades wave quantization (e.g. 172 vs 230
 // tiles at M = 512) against per-tile efficiency and knows nothing of the
-// epilogue's bytes, which count at a short K.  Narrow outputs (Wo) and long K (W2) use stream-K
-// instead, when every block gets at least two 32-wide k-iterations.  *cost: the
-// pick's estimate (per unit of K).
-int tile_pick(int M, int N, float* cost) {
+// epilogue's bytes, which count at a short K.  Two rounds of 256x256 and three of
+// 256x128 come out even (257 - 384 tiles of 256x256, whose second round is at
+// most half full); the three rounds measure faster: logits 3072 x 8192 x 1024 82 ->
+// 70 us, x 3072 171 -> 145, W2 6144 x 4096 x 11008 503 -> 470, QKV 3200 x 7680 x
+// 2560 157 -> 143.  Token-major operands take 256x256 there (forward + backward
+// 3072 wide, 768 - 8192 tokens, 1 - 4% faster: the smaller tile pays more
+// transposing reads).  Narrow outputs (Wo) and long K (W2) use stream-K instead,
+// when every block gets at least two 32-wide k-iterations.  *cost: the pick's
+// estimate (per unit of K).
+int tile_pick(int M, int N, bool tokens, float* cost) {
     struct Cand { int cfg, bn, bm; float rate; };
-    constexpr Cand dp[] = {{GCFG_D8_256x256, 256, 256, 5.0f}, {GCFG_D8_192x256, 192, 256, 4.35f},
-                           {GCFG_D8_256x128, 256, 128, 3.75f}, {GCFG_D8_192x128, 192, 128, 3.7f},
+    constexpr Cand dp[] = {{GCFG_D8_256x128, 256, 128, 3.75f}, {GCFG_D8_256x256, 256, 256, 5.0f},
+                           {GCFG_D8_192x256, 192, 256, 4.35f}, {GCFG_D8_192x128, 192, 128, 3.7f},
                            {GCFG_D8_128x128, 128, 128, 3.0f}};
     float best = 3.0e38f;
     int cfg = 0;
     for (const Cand& c : dp) {
         const long long tiles = (long long)((N + c.bn - 1) / c.bn) * ((M + c.bm - 1) / c.bm);
         const float t = (float)((tiles + SK_P - 1) / SK_P) * (float)c.bn * (float)c.bm / c.rate;
-        if (t < best) { best = t; cfg = c.cfg; }
+        if (t < best || (tokens && t == best && c.cfg == GCFG_D8_256x256)) { best = t; cfg = c.cfg; }
     }
     if (cost) *cost = best;
     return cfg;
@@ -945,7 +951,7 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
             // faster (15.3 + 8.5 us stream-K + fix-up against one 17.5 us round)
             cfg = GCFG_D8_128x128_SK;
         } else {
-            cfg = tile_pick(a.M, a.N, nullptr);
+            cfg = tile_pick(a.M, a.N, false, nullptr);
         }
     }
     // The 8-wave 192x256, 192x128 and 128x128 tiles run the 16x16x32 form: at
@@ -1000,7 +1006,7 @@ hipError_t launch_tokens(const GemmArgs& a, hipStream_t st) {
         hipLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_DP>), dim3(tiles), dim3(Tl::NT), 0, st, a, 1, 0LL);
         return hipGetLastError();
     };
-    switch (a.force_cfg ? a.force_cfg : tile_pick(a.M, a.N, nullptr)) {
+    switch (a.force_cfg ? a.force_cfg : tile_pick(a.M, a.N, true, nullptr)) {
         case GCFG_D8_256x256: return go(PTile<2, 4, 8, 4, 1, 4, true>{});
         case GCFG_D8_256x128: return go(PTile<4, 2, 4, 4, 2, 3, true>{});
         case GCFG_D8_192x256: return go(DTile<2, 4, 3, 2, true, 4, true>{});
@@ -1075,7 +1081,7 @@ hipError_t launch_gemm_resid_norm(const GemmArgs& a, const float* gamma, float e
 
 float gemm_tile_cost(int M, int N) {
     float c = 0.f;
-    (void)tile_pick(M, N, &c);
+    (void)tile_pick(M, N, true, &c);
     return c;
 }
 
