@@ -768,24 +768,30 @@ __global__ __launch_bounds__(Tl::NT) void gemm_fixup_kernel(GemmArgs a, int P, l
 }
 
 template <class Tl, int EPI>
+hipError_t launch_dp(const GemmArgs& a, hipStream_t st) {
+    const int tiles = ((a.N + Tl::BN - 1) / Tl::BN) * ((a.M + Tl::BM - 1) / Tl::BM);
+    const long long T = (long long)tiles * (a.K / Tl::KI);
+    if (a.prof_start)
+        hipExtLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_DP>), dim3(tiles), dim3(Tl::NT), 0, st, a.prof_start,
+                              a.prof_stop, 0u, a, 1, T);
+    else
+        hipLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_DP>), dim3(tiles), dim3(Tl::NT), 0, st, a, 1, T);
+    return hipGetLastError();
+}
+
+template <class Tl, int EPI>
 hipError_t launch_tile(const GemmArgs& a, bool sk, hipStream_t st) {
+    if (!sk) return launch_dp<Tl, EPI>(a, st);
     const int nbN = (a.N + Tl::BN - 1) / Tl::BN, nbM = (a.M + Tl::BM - 1) / Tl::BM;
     const int tiles = nbN * nbM;
     const long long T = (long long)tiles * (a.K / Tl::KI);
-    if (sk) {
-        if (!a.sk_part || (size_t)SK_P * 2 * Tl::BN * Tl::BM > a.sk_part_floats) return hipErrorInvalidValue;
-        if (a.prof_start && hipEventRecord(a.prof_start, st) != hipSuccess) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_SK>), dim3(SK_P), dim3(Tl::NT), 0, st, a, SK_P, T);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL((gemm_fixup_kernel<Tl, EPI>), dim3(tiles, Tl::FTN), dim3(Tl::NT), 0, st, a, SK_P, T);
-        if (a.prof_stop && hipEventRecord(a.prof_stop, st) != hipSuccess) return hipErrorInvalidValue;
-    } else if (a.prof_start) {
-        hipExtLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_DP>), dim3(tiles), dim3(Tl::NT), 0, st, a.prof_start,
-                              a.prof_stop, 0u, a, 1, T);
-    } else {
-        hipLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_DP>), dim3(tiles), dim3(Tl::NT), 0, st, a, 1, T);
-    }
+    if (!a.sk_part || (size_t)SK_P * 2 * Tl::BN * Tl::BM > a.sk_part_floats) return hipErrorInvalidValue;
+    if (a.prof_start && hipEventRecord(a.prof_start, st) != hipSuccess) return hipErrorInvalidValue;
+    hipLaunchKernelGGL((gemm_kernel<Tl, EPI, MODE_SK>), dim3(SK_P), dim3(Tl::NT), 0, st, a, SK_P, T);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL((gemm_fixup_kernel<Tl, EPI>), dim3(tiles, Tl::FTN), dim3(Tl::NT), 0, st, a, SK_P, T);
+    if (a.prof_stop && hipEventRecord(a.prof_stop, st) != hipSuccess) return hipErrorInvalidValue;
     return hipGetLastError();
 }
 
@@ -952,6 +958,11 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
             cfg = GCFG_D8_128x128_SK;
         } else {
             cfg = tile_pick(a.M, a.N, false, nullptr);
+            // Of 8 - 16 stages of 64 k the ping-pong tile's longer ramp is too
+            // large a share.  us, DTile | ping-pong: logits 256 x 32000 x 512 16.5 |
+            // 20.6, 256 x 32000 x 768 20 | 24, 1024 x 8192 x 768 20 | 23, 200 x 32000
+            // x 1024 24 | 26.6; K = 1536 34.0 | 34.9, K = 2048 even, more: slower.
+            if (cfg == GCFG_D8_256x128 && a.K <= 1024) cfg = GCFG_DT_256x128;
         }
     }
     // The 8-wave 192x256, 192x128 and 128x128 tiles run the 16x16x32 form: at
@@ -969,6 +980,7 @@ hipError_t launch_epi(const GemmArgs& a, hipStream_t st) {
         case GCFG_D4_128x128_SK: return launch_tile<DTile<2, 2, 2, 2>, EPI>(a, true, st);
         case GCFG_D8_256x128: return launch_tile<Tile256x128, EPI>(a, false, st);
         case GCFG_D8_256x128_SK: return launch_tile<Tile256x128, EPI>(a, true, st);
+        case GCFG_DT_256x128: return launch_dp<DTile<4, 2, 2, 2, true>, EPI>(a, st);
         case GCFG_D4_256x256: return launch_tile<DTile<2, 2, 4, 4>, EPI>(a, false, st);
         case GCFG_D4_256x256_SK: return launch_tile<DTile<2, 2, 4, 4>, EPI>(a, true, st);
         case GCFG_D4_256x128: return launch_tile<DTile<2, 2, 4, 2>, EPI>(a, false, st);

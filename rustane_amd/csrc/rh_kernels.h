@@ -77,6 +77,7 @@ enum GemmCfg {
     GCFG_D8_192x128_SK = 25,
     GCFG_D8_128x128 = 26,    // 8 waves (64x32 each), 16x16x32 MFMA
     GCFG_D8_128x128_SK = 27,
+    GCFG_DT_256x128 = 28,    // 8 waves (64x64 each), 16x16x32 MFMA, no ping-pong
 };
 // Few tokens (rh_skinny.hip): every weight row streamed once for all M <=
 // SKINNY_M tokens.  launch_gemm_skinny: EPI_F32, EPI_SWIGLU, EPI_QKV;

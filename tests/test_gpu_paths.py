@@ -54,6 +54,23 @@ def test_ping_pong_step_counts(lib, name, K):  # noqa: F811
     close(out, y, 1e-5, f"{name} K {K}")
 
 
+# The 256x128 tile without ping-pong, which short k loops take: plain and SwiGLU
+# stores with ragged rows and columns and 4 - 32 k steps, and picked by size (one
+# round of 252 tiles) at the last K that takes it and the first that does not.
+@pytest.mark.parametrize("cfg,M,N,K", [(28, 270, 520, 128), (28, 129, 1000, 640), (28, 128, 256, 1024),
+                                       (0, 192, 32004, 1024), (0, 192, 32004, 1152)])
+def test_short_k_tile(lib, cfg, M, N, K):  # noqa: F811
+    x, w, y = operands(28, M, N, K)
+    out = np.full((M, N), np.nan, np.float32)
+    run(lib, EPI_F32, cfg, x, w, io=out)
+    close(out, y, 1e-5, f"store {M} {N} {K}")
+    F = N // 256 * 128
+    if F:
+        out16 = np.zeros(up16(M) * F, np.float16)
+        run(lib, EPI_SWIGLU, cfg, x, np.ascontiguousarray(w[:2 * F]), out16=out16)
+        close(frag_unpack(out16, M, F), swiglu_ref(y[:, :2 * F])[0], 2e-3, "swiglu")
+
+
 # Few tokens: token tiles of 16 full and ragged, 64 and the first count past
 # it; every choice of row tiles per block (by N), ragged in N; fewer k chunks
 # than waves, more, and a remainder.  fp32 sums of K <= 1408 products: 1e-5 of
