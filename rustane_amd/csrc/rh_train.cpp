@@ -471,9 +471,11 @@ int enqueue_backward(rh_ctx* ctx, int B, int S, float loss_scale, int nuniq) {
     // tile kernels read the token-major activations and their gradients in place
     // (then read[g] is the GEMM's end); otherwise the rows past the last token
     // have to be zeros and the GEMMs take padded token-inner copies.  From 1000
-    // tokens on that is 1 - 6% of a pass at every width (512 - 4096; 20 layers of
-    // 4096, 8 x 512 accumulated: 98.2 -> 95.3 ms), at 128 - 512 tokens 7% (2304
-    // wide) to -5% (512 wide).  The store-wave kernel keeps the copies: two
+    // tokens on that is 1 - 6% of a pass at nearly every width (512 - 4096; 20
+    // layers of 4096, 8 x 512 accumulated: 98.2 -> 95.3 ms), at 128 - 768 tokens -3
+    // to 8% at 512 - 4096 wide; a chain of the smallest kernels loses, since the
+    // main stream then waits for the product instead of its copy (8 layers, 128
+    // tokens: 512 wide 8%, 128 wide 12%).  The store-wave kernel keeps the copies: two
     // transposing reads for each of its 128x128 tile's operands take 4096 x
     // 11008 x 512 from 72 to 93 us beside the other stream (20 layers of 4096
     // after a zero, 1 x 512: 19.7 ms in place, 18.7 with copies).
